@@ -30,6 +30,7 @@
 #include "lusgs.hpp"
 #include "mstcfd.h"
 #include "prep.hpp"
+#include "transfer.hpp"
 
 using namespace mstk;
 
@@ -506,6 +507,8 @@ struct mst_batch {
     int32_t *ci0 = nullptr, *ci1 = nullptr;
     double *part = nullptr;
     int *cnt = nullptr, *bad = nullptr;
+    int32_t *cnew = nullptr;  // device position of each file cell, case after case
+    Transfer link;            // host states in file order
     int iold = 0, inew = 1;
     bool dt_valid = false;
     bool shadow_ok[4] = {false, false, false, false};
@@ -575,10 +578,11 @@ void release(mst_batch *b) {
                     b->inc_code, b->inc_w, b->inc_n, b->inc_dx, b->inc_w32, b->inc_n32, b->inc_dx32, b->ivol32,
                     b->pstart, b->pface, b->pfi, b->ploc, b->hstart, b->hcell, b->hloc, b->lu_cells, b->lu_nb,
                     b->lu_face, b->lu_pcase, b->lu_fcase, b->lu_n, b->lu_r, b->lu_D, b->lu_dQ, b->lu_cstart,
-                    b->lu_active};
+                    b->lu_active, b->cnew};
     for (void *p : bufs)
         if (p) (void)hipFree(p);
     b->hg.release();
+    b->link.release();
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
 }
@@ -1434,6 +1438,7 @@ int mst_batch_create(int n_cases, const mst_mesh *const *meshes, const mst_confi
     std::vector<int32_t> fc0(b->NF), fc1(b->NF), finfo(b->NF), ell((size_t)b->slots * b->NC, -1), scheme(n_cases);
     std::vector<double> fn(b->NF * dim), fxf(b->NF * dim), feta(b->NF), cvol(b->NC), cxc(b->NC * dim),
         cshalf(b->NC * dim), gam(n_cases), cflv(n_cases), ncells(n_cases);
+    std::vector<int32_t> cnew(b->NC);
     std::vector<int32_t> inc_code((size_t)b->slots * b->NC, -2), frec0(b->NF, -1), frec1(b->NF, -1);
     std::vector<double> inc_w((size_t)b->slots * b->NC, 0.0), inc_n((size_t)b->slots * b->NC * dim, 0.0),
         inc_dx((size_t)b->slots * b->NC * dim, 0.0);
@@ -1459,6 +1464,7 @@ int mst_batch_create(int n_cases, const mst_mesh *const *meshes, const mst_confi
         }
         if ((c.compat & MST_COMPAT_GRAD_LASTINT) && P.quirk_face >= 0) feta[fs + P.quirk_face] = 1.0;
         for (int64_t k = 0; k < P.nc; k++) {
+            cnew[cs + k] = (int32_t)(cs + P.cell_new_of_old[k]);
             cvol[cs + k] = P.cvol[k];
             for (int d = 0; d < dim; d++) {
                 cxc[(cs + k) * dim + d] = P.cxc[k * dim + d];
@@ -1498,6 +1504,7 @@ int mst_batch_create(int n_cases, const mst_mesh *const *meshes, const mst_confi
         gam[i] = c.gamma;
         cflv[i] = c.cfl;
         ncells[i] = (double)P.nc;
+        b->link.most = std::max(b->link.most, P.nc * nv);
     }
 #define TRY(e)            \
     do {                  \
@@ -1528,6 +1535,7 @@ int mst_batch_create(int n_cases, const mst_mesh *const *meshes, const mst_confi
     TRY(dupload(&b->cvol, cvol));
     TRY(dupload(&b->cxc, cxc));
     TRY(dupload(&b->cshalf, cshalf));
+    TRY(dupload(&b->cnew, cnew));
     TRY(dupload(&b->inc_code, inc_code));
     TRY(dupload(&b->inc_w, inc_w));
     TRY(dupload(&b->inc_n, inc_n));
@@ -1611,16 +1619,12 @@ int mst_batch_set_state(mst_batch *b, int case_id, const double *Q, int64_t n_ce
     if (case_id < 0 || case_id >= b->n || !Q) return mst::fail(MST_E_ARG, "bad case");
     const mst::Prepared &P = b->preps[case_id];
     if (n_cells != P.nc) return mst::fail(MST_E_ARG, "state size does not match the case's mesh");
-    const int nv = b->nv;
-    std::vector<double> buf(P.nc * nv);
-    for (int64_t i = 0; i < P.nc; i++)
-        for (int k = 0; k < nv; k++) buf[i * nv + k] = Q[(int64_t)P.cell_old_of_new[i] * nv + k];
-    HIPCHK(hipStreamSynchronize(b->stream));
     // an inactive case keeps its state in every buffer (the buffers rotate under it)
+    double *dst[4];
+    int nd = 0;
     for (int i = 0; i < 4; i++)
-        if (i == b->iold || !b->active[case_id])
-            HIPCHK(hipMemcpy(b->Q[i] + b->cstart[case_id] * nv, buf.data(), sizeof(double) * buf.size(),
-                             hipMemcpyHostToDevice));
+        if (i == b->iold || !b->active[case_id]) dst[nd++] = b->Q[i];
+    HIPCHK(b->link.put(b->stream, P.nc, b->nv, b->cnew + b->cstart[case_id], Q, dst, nd));
     for (int i = 0; i < 4; i++) b->shadow_ok[i] = false;
     b->dt_valid = false;
     return MST_OK;
@@ -1631,13 +1635,7 @@ int mst_batch_get_state(mst_batch *b, int case_id, double *Q, int64_t n_cells) {
     if (case_id < 0 || case_id >= b->n || !Q) return mst::fail(MST_E_ARG, "bad case");
     const mst::Prepared &P = b->preps[case_id];
     if (n_cells != P.nc) return mst::fail(MST_E_ARG, "state size does not match the case's mesh");
-    const int nv = b->nv;
-    std::vector<double> buf(P.nc * nv);
-    HIPCHK(hipStreamSynchronize(b->stream));
-    HIPCHK(hipMemcpy(buf.data(), b->Q[b->iold] + b->cstart[case_id] * nv, sizeof(double) * buf.size(),
-                     hipMemcpyDeviceToHost));
-    for (int64_t c = 0; c < P.nc; c++)
-        for (int k = 0; k < nv; k++) Q[c * nv + k] = buf[(int64_t)P.cell_new_of_old[c] * nv + k];
+    HIPCHK(b->link.fetch(b->stream, P.nc, b->nv, b->cnew + b->cstart[case_id], b->Q[b->iold], Q));
     return MST_OK;
 }
 

@@ -17,6 +17,7 @@
 #include "mlp.hpp"
 #include "mstcfd.h"
 #include "prep.hpp"
+#include "transfer.hpp"
 
 namespace mst {
 const std::string &last_error();
@@ -103,6 +104,8 @@ struct mst_ctx {
     double *fin_mid = nullptr;  // first-level results of the two-level finish
     bool dt_valid = false;   // scal[0] holds the CFL time step of the current Old state
     int *bad = nullptr;
+    int32_t *cnew = nullptr;  // device position of each file cell
+    Transfer link;            // host states in file order
     bool viscous = false;     // mu or kappa > 0: the face strategy with the viscous kernels
     double *gw = nullptr;     // viscous: per cell Green-Gauss gradients of (u, T), [nc][dim + 1][dim]
     // LU-SGS steady driver (built on first use): cell colours, the cells of each colour in ascending
@@ -836,10 +839,11 @@ void release(mst_ctx *x) {
                     x->scal, x->part, x->fin_mid, x->bad, x->Q32[0], x->Q32[1], x->Q32[2], x->Q32[3], x->rec32,
                     x->frec0, x->frec1, x->inc_code, x->inc_w, x->inc_n, x->inc_dx, x->inc_w32, x->inc_n32,
                     x->inc_dx32, x->ivol32, x->pstart, x->pface, x->pfi, x->ploc, x->hstart, x->hcell, x->hloc,
-                    x->lu_cells, x->lu_nb, x->lu_face, x->lu_n, x->lu_r, x->lu_D, x->lu_dQ, x->gw};
+                    x->lu_cells, x->lu_nb, x->lu_face, x->lu_n, x->lu_r, x->lu_D, x->lu_dQ, x->gw, x->cnew};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     x->hg.release();
+    x->link.release();
     for (int k = 0; k < MST_K_COUNT; k++)
         for (auto &pr : x->ev[k]) {
             (void)hipEventDestroy(pr.first);
@@ -850,22 +854,8 @@ void release(mst_ctx *x) {
     delete x;
 }
 
-int permute_in(const mst_ctx *x, const double *Q, std::vector<double> &buf) {
-    const int nv = x->nv;
-    buf.resize(x->nc * nv);
-    const auto &old_of_new = x->prep.P.cell_old_of_new;
-    for (int64_t i = 0; i < x->nc; i++)
-        for (int k = 0; k < nv; k++) buf[i * nv + k] = Q[(int64_t)old_of_new[i] * nv + k];
-    return MST_OK;
-}
-
 int fetch_cells(mst_ctx *x, const double *dsrc, int width, double *out) {
-    std::vector<double> buf(x->nc * width);
-    HIPCHK(hipStreamSynchronize(x->stream));
-    HIPCHK(hipMemcpy(buf.data(), dsrc, sizeof(double) * buf.size(), hipMemcpyDeviceToHost));
-    const auto &new_of_old = x->prep.P.cell_new_of_old;
-    for (int64_t c = 0; c < x->nc; c++)
-        for (int k = 0; k < width; k++) out[c * width + k] = buf[(int64_t)new_of_old[c] * width + k];
+    HIPCHK(x->link.fetch(x->stream, x->nc, width, x->cnew, dsrc, out));
     return MST_OK;
 }
 
@@ -1220,6 +1210,8 @@ int mst_ctx_create(const mst_mesh *m, const mst_config *cfg, mst_ctx **out) {
     TRY(dupload(&x->cvol, P.cvol));
     TRY(dupload(&x->cxc, P.cxc));
     TRY(dupload(&x->cshalf, P.cshalf));
+    TRY(dupload(&x->cnew, P.cell_new_of_old));
+    x->link.most = x->nc * x->nv;
     for (int i = 0; i < 4; i++) TRY(dalloc(&x->Q[i], x->nc * x->nv));
     TRY(dalloc(&x->G, x->nf * x->nv));
     TRY(dalloc(&x->rec, (int64_t)x->slots * x->nc * x->nv));
@@ -1263,10 +1255,7 @@ const mst_prep *mst_ctx_prep(const mst_ctx *ctx) { return ctx ? &ctx->prep : nul
 int mst_set_state(mst_ctx *ctx, const double *Q, int64_t n_cells) {
     CTX_GUARD(ctx);
     if (!Q || n_cells != ctx->nc) return mst::fail(MST_E_ARG, "state size does not match the mesh");
-    std::vector<double> buf;
-    permute_in(ctx, Q, buf);
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    HIPCHK(hipMemcpy(ctx->Q[ctx->iold], buf.data(), sizeof(double) * buf.size(), hipMemcpyHostToDevice));
+    HIPCHK(ctx->link.put(ctx->stream, ctx->nc, ctx->nv, ctx->cnew, Q, &ctx->Q[ctx->iold], 1));
     ctx->shadow_ok[ctx->iold] = false;
     ctx->dt_valid = false;
     return MST_OK;
