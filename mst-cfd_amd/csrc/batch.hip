@@ -152,7 +152,7 @@ __global__ __launch_bounds__(NT) void kb_update(const BArgs<T> a) {
 #pragma unroll
                 for (int k = 0; k < NV; k++) r[k] += cmp[k];
             }
-            stage_cell<NV, F32>(ua, c, r, red, L2, DT);
+            stage_cell<NV, F32>(ua, c, ua.dt[0], r, red, L2, DT);
         }
         if (L2) {
             double v[NV];
@@ -199,7 +199,7 @@ __global__ __launch_bounds__(NT) void kb_cell(const BArgs<T> a) {
 #pragma unroll
                 for (int k = 0; k < NV; k++) r[k] += cmp[k];
             }
-            stage_cell<NV, F32>(ua, c, r, red, L2, DT);
+            stage_cell<NV, F32>(ua, c, ua.dt[0], r, red, L2, DT);
         }
         if (L2) {
             double v[NV];
@@ -263,7 +263,7 @@ __global__ __launch_bounds__(BLOCK) void kb_patch(const BArgs<T> a, const PatchA
             for (int s = 0; s < MAXF; s++) cl[s] = p.loc[(int64_t)s * ua.nc + c];
             double r[NV];
             patch_sum<NV, MAXF, F32>(gsh, npf, cl, r);
-            stage_cell<NV, F32>(ua, c, r, red, L2, DT);
+            stage_cell<NV, F32>(ua, c, ua.dt[0], r, red, L2, DT);
         }
         if (L2) {
             double v[NV];
@@ -321,7 +321,7 @@ __global__ __launch_bounds__(BLOCK, (kb_fused_waves<DIM, T, MAXF>())) void kb_fu
         if (c < I.end) {
             double r[NV];
             patch_sum<NV, MAXF, F32>(L.g, L.npf, cl, r);
-            stage_cell<NV, F32>(ua, c, r, red, L2, DT);
+            stage_cell<NV, F32>(ua, c, ua.dt[0], r, red, L2, DT);
         }
         if (L2) {
             double v[NV];

@@ -438,7 +438,9 @@ struct UpdArgs {
     const double *__restrict__ Qn;
     const double *__restrict__ vol;
     const double *__restrict__ sh;  // half sums of |S_d| per cell (CFL)
-    const double *__restrict__ dt;  // [0] dt of this stage
+    const double *__restrict__ dt;  // [0] dt of this stage, when dt_n == 0; else it is the minimum of
+    const double *__restrict__ dt_part;  // dt_part[0..dt_n), the previous step's block minima
+    int dt_n;
     double ca, cb;
     int stage0;
     // mixed form (FP32 kernels read only the FP32 shadow, so an intermediate stage's FP64 state is
@@ -566,6 +568,24 @@ struct StageIn {
     double sh[NV - 2];  // the cell's CFL half-sums, on a launch that reduces the time step
 };
 
+// The time step of the stage, the same in every lane; the whole wave must be active.  Each wave takes the minimum of
+// the block minima itself (a minimum does not depend on the order), with its loads in flight together: on
+// meshes of few blocks that costs less than a launch between two steps (STEP_DT_MAX in solver.hip).
+__device__ __forceinline__ double stage_dt(const UpdArgs &a) {
+    if (a.dt_n == 0) return a.dt[0];
+    double v = INFINITY;
+    for (int i = threadIdx.x & 63; i < a.dt_n; i += 8 * 64) {
+        double x[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) x[u] = a.dt_part[i + 64 * u < a.dt_n ? i + 64 * u : i];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v = fmin(v, x[u]);
+    }
+    for (int m = 32; m > 0; m >>= 1) v = fmin(v, __shfl_xor(v, m, 64));
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),  // (a scalar: no vector registers)
+                            __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+
 template <int NV, bool F32>
 __device__ __forceinline__ void stage_load(const UpdArgs &a, int64_t c, StageIn<NV> &in) {
     in.V = a.vol[c];
@@ -579,11 +599,11 @@ __device__ __forceinline__ void stage_load(const UpdArgs &a, int64_t c, StageIn<
 }
 
 template <int NV, bool F32>
-__device__ __forceinline__ void stage_cell(const UpdArgs &a, int64_t c, const StageIn<NV> &in, const double (&r)[NV],
+__device__ __forceinline__ void stage_cell(const UpdArgs &a, int64_t c, double dt, const StageIn<NV> &in, const double (&r)[NV],
                                            double (&red)[NV + 1], const bool L2, const bool DT) {
     constexpr int DIM = NV - 2;
     const double V = in.V;
-    const double dtv = a.dt[0] / V;
+    const double dtv = dt / V;
     const bool pre = F32 && a.pre;
     double out[NV];
     if (pre) {  // Qs = ca Q^n + cb Q_s (cb = 1 on the first stage: the same arithmetic as below)
@@ -613,7 +633,7 @@ __device__ __forceinline__ void stage_cell(const UpdArgs &a, int64_t c, const St
         const double p = (out[NV - 1] - 0.5 * ke / out[0]) * (a.gamma - 1);
         if (!(out[0] > 0) || !(p > 0)) a.bad[0] = 1;
     }
-    if (!(a.dt[0] > 0)) a.bad[0] = 1;  // a NaN or non-physical state gave no positive CFL time step
+    if (!(dt > 0)) a.bad[0] = 1;  // a NaN or non-physical state gave no positive CFL time step
     if (L2) {
         const double iV = frcp(V);
 #pragma unroll
@@ -626,19 +646,20 @@ __device__ __forceinline__ void stage_cell(const UpdArgs &a, int64_t c, const St
 }
 
 template <int NV, bool F32>
-__device__ __forceinline__ void stage_cell(const UpdArgs &a, int64_t c, const double (&r)[NV], double (&red)[NV + 1],
-                                           const bool L2, const bool DT) {
+__device__ __forceinline__ void stage_cell(const UpdArgs &a, int64_t c, double dt, const double (&r)[NV],
+                                           double (&red)[NV + 1], const bool L2, const bool DT) {
     StageIn<NV> in;
     stage_load<NV, F32>(a, c, in);
-    stage_cell<NV, F32>(a, c, in, r, red, L2, DT);
+    stage_cell<NV, F32>(a, c, dt, in, r, red, L2, DT);
 }
 
 // stage_cell for the lanes of one block, then the block's partials of |R/V|^2 and the CFL time step.
 // Every lane of the block must call it (block-level reductions).
 // lds (DYN): NV * BLOCK / 64 doubles of the kernel's dynamic LDS for the reductions, in place of a static
 // array (which would count against every block's LDS for the whole kernel).
-template <int NV, bool STAGE, bool F32, bool DYN = false>
-__device__ __forceinline__ void stage_tail(const UpdArgs &a, int64_t c, bool valid, const double (&r)[NV],
+// dt: stage_dt (unused by a residual-only evaluation).  in: the inputs when they are loaded already.
+template <int NV, bool STAGE, bool F32, int NT = BLOCK, bool DYN = false>
+__device__ __forceinline__ void stage_tail(const UpdArgs &a, int64_t c, bool valid, double dt, const double (&r)[NV],
                                            int64_t blk, const bool L2, const bool DT, const StageIn<NV> *in = nullptr,
                                            double *lds = nullptr) {
     if constexpr (!STAGE) {
@@ -655,7 +676,7 @@ __device__ __forceinline__ void stage_tail(const UpdArgs &a, int64_t c, bool val
                     v[k] = x * x;
                 }
             }
-            block_partial<NV, false>(v, a.part_l2 + blk, gridDim.x);
+            block_partial<NV, false, NT>(v, a.part_l2 + blk, gridDim.x);
         }
         return;
     } else {
@@ -665,25 +686,25 @@ __device__ __forceinline__ void stage_tail(const UpdArgs &a, int64_t c, bool val
         red[NV] = INFINITY;
         if (valid) {
             if (in)
-                stage_cell<NV, F32>(a, c, *in, r, red, L2, DT);
+                stage_cell<NV, F32>(a, c, dt, *in, r, red, L2, DT);
             else
-                stage_cell<NV, F32>(a, c, r, red, L2, DT);
+                stage_cell<NV, F32>(a, c, dt, r, red, L2, DT);
         }
         if (L2) {  // uniform over the launch
             double v[NV];
 #pragma unroll
             for (int k = 0; k < NV; k++) v[k] = red[k];
             if constexpr (DYN)
-                block_partial<NV, false>(v, a.part_l2 + blk, gridDim.x, lds);
+                block_partial<NV, false, NT>(v, a.part_l2 + blk, gridDim.x, lds);
             else
-                block_partial<NV, false>(v, a.part_l2 + blk, gridDim.x);
+                block_partial<NV, false, NT>(v, a.part_l2 + blk, gridDim.x);
         }
         if (DT) {
             double v[1] = {red[NV]};
             if constexpr (DYN)
-                block_partial<1, true>(v, a.part_dt + blk, 1, lds);
+                block_partial<1, true, NT>(v, a.part_dt + blk, 1, lds);
             else
-                block_partial<1, true>(v, a.part_dt + blk, 1);
+                block_partial<1, true, NT>(v, a.part_dt + blk, 1);
         }
     }
 }
@@ -695,6 +716,7 @@ __global__ __launch_bounds__(BLOCK) void k_update(const UpdArgs a) {
     const int64_t blk = block_id();
     const int64_t c = blk * BLOCK + threadIdx.x;
     const bool valid = c < a.nc;
+    const double dt = (MODE & UPD_STAGE) ? stage_dt(a) : 0.0;
     double r[NV], cmp[NV];
 #pragma unroll
     for (int k = 0; k < NV; k++) r[k] = cmp[k] = 0;
@@ -712,7 +734,7 @@ __global__ __launch_bounds__(BLOCK) void k_update(const UpdArgs a) {
             for (int k = 0; k < NV; k++) r[k] += cmp[k];
         }
     }
-    stage_tail<NV, (MODE & UPD_STAGE) != 0, F32>(a, c, valid, r, blk, (MODE & UPD_L2) != 0, (MODE & UPD_DT) != 0);
+    stage_tail<NV, (MODE & UPD_STAGE) != 0, F32>(a, c, valid, dt, r, blk, (MODE & UPD_L2) != 0, (MODE & UPD_DT) != 0);
 }
 
 // Sum over cell c's faces of +-G_f (accumulate: c0 adds, c1 subtracts), slots in order.  The face
@@ -788,6 +810,7 @@ __global__ __launch_bounds__(BLOCK) void k_cell(const FluxArgs<T> fa, const UpdA
     const int64_t blk = block_id();
     const int64_t c = blk * BLOCK + threadIdx.x;
     const bool valid = c < a.nc;
+    const double dt = stage_dt(a);
     double r[NV], cmp[NV];
 #pragma unroll
     for (int k = 0; k < NV; k++) r[k] = cmp[k] = 0;
@@ -798,7 +821,7 @@ __global__ __launch_bounds__(BLOCK) void k_cell(const FluxArgs<T> fa, const UpdA
             for (int k = 0; k < NV; k++) r[k] += cmp[k];
         }
     }
-    stage_tail<NV, true, F32>(a, c, valid, r, blk, a.l2, a.dtred);
+    stage_tail<NV, true, F32>(a, c, valid, dt, r, blk, a.l2, a.dtred);
 }
 
 // ------------------------------------------------------------------------------------ patch strategy
@@ -885,16 +908,17 @@ __device__ __forceinline__ void patch_sum(const double *g, int npf, const int (&
     }
 }
 
-// STAGE false: the residual only (R and, with a.l2, its norms), for the implicit steady driver
-template <int DIM, int SCHEME, bool SECOND, typename T, int MAXF, bool STAGE = true>
-__global__ __launch_bounds__(BLOCK) void k_patch(const FluxArgs<T> fa, const UpdArgs a, const PatchArgs p) {
+// STAGE false: the residual only (R and, with a.l2, its norms), for the implicit steady driver.  NT lanes per patch of
+// BLOCK cells: twice as many on meshes of few patches, where the patch's faces then take one pass.
+template <int DIM, int SCHEME, bool SECOND, typename T, int MAXF, bool STAGE = true, int NT = BLOCK>
+__global__ __launch_bounds__(NT) void k_patch(const FluxArgs<T> fa, const UpdArgs a, const PatchArgs p) {
     constexpr int NV = DIM + 2;
     constexpr bool F32 = std::is_same<T, float>::value;
     extern __shared__ double gsh[];  // NV x npf, component-major: consecutive lanes, consecutive banks
     const int64_t blk = block_id();
     const int32_t f0 = p.start[blk];
     const int npf = p.start[blk + 1] - f0;
-    for (int i = threadIdx.x; i < npf; i += BLOCK) {
+    for (int i = threadIdx.x; i < npf; i += NT) {
         int64_t f;
         int info;
         patch_face(p, fa.finfo, f0 + i, f, info);
@@ -903,15 +927,16 @@ __global__ __launch_bounds__(BLOCK) void k_patch(const FluxArgs<T> fa, const Upd
 #pragma unroll
         for (int k = 0; k < NV; k++) gsh[k * npf + i] = g[k];
     }
+    const double dt = STAGE ? stage_dt(a) : 0.0;
     __syncthreads();
     const int64_t c = blk * BLOCK + threadIdx.x;
-    const bool valid = c < a.nc;
+    const bool valid = (NT == BLOCK || threadIdx.x < BLOCK) && c < a.nc;
     int cl[MAXF];
 #pragma unroll
     for (int s = 0; s < MAXF; s++) cl[s] = valid ? p.loc[(int64_t)s * a.nc + c] : -1;  // padded to MAXF rows
     double r[NV];
     patch_sum<NV, MAXF, F32>(gsh, npf, cl, r);
-    stage_tail<NV, STAGE, F32>(a, c, valid, r, blk, a.l2, a.dtred);
+    stage_tail<NV, STAGE, F32, NT>(a, c, valid, dt, r, blk, a.l2, a.dtred);
 }
 
 // Order 2 in one kernel: the patch also computes the limited gradients of its own cells and of its
@@ -1062,8 +1087,8 @@ inline size_t fused_lds_bytes(int dim, int nv, int max_pf, bool f32, bool staged
 // each record once per patch; the inputs of every face's solve are the records k_flux would read, so
 // the results are bit-identical.  LDS: the fused kernel's FP32 layout, 8 * NV bytes per face (the
 // size of the FP64 fluxes that overwrite them).
-template <int DIM, int SCHEME, int MAXF>
-__global__ __launch_bounds__(BLOCK) void k_patch_rec(const FluxArgs<float> fa, const UpdArgs a, const PatchArgs p,
+template <int DIM, int SCHEME, int MAXF, int NT = BLOCK>
+__global__ __launch_bounds__(NT) void k_patch_rec(const FluxArgs<float> fa, const UpdArgs a, const PatchArgs p,
                                                      const HaloArgs h) {
     constexpr int NV = DIM + 2;
     extern __shared__ double gsh[];
@@ -1072,7 +1097,7 @@ __global__ __launch_bounds__(BLOCK) void k_patch_rec(const FluxArgs<float> fa, c
     const int npf = p.start[blk + 1] - f0;
     FusedLds<float> L(gsh, npf, NV);
     const int64_t c = blk * BLOCK + threadIdx.x;
-    const bool valid = c < a.nc;
+    const bool valid = (NT == BLOCK || threadIdx.x < BLOCK) && c < a.nc;
     int cl[MAXF];
 #pragma unroll
     for (int s = 0; s < MAXF; s++) cl[s] = valid ? p.loc[(int64_t)s * a.nc + c] : -1;
@@ -1087,7 +1112,9 @@ __global__ __launch_bounds__(BLOCK) void k_patch_rec(const FluxArgs<float> fa, c
 #pragma unroll
         for (int k = 0; k < NV; k++) L.r(l & 1, k, l >> 1, NV) = q[k];
     }
-    for (int j = threadIdx.x; j < nh; j += BLOCK) {
+    // (lanes past the patch's cells take the halo beside them)
+    for (int j = NT > BLOCK ? (int)threadIdx.x - BLOCK : threadIdx.x; j < nh; j += NT > BLOCK ? NT - BLOCK : BLOCK) {
+        if (NT > BLOCK && j < 0) break;
         const int64_t hc = h.cell[h0 + j];
 #pragma unroll
         for (int s = 0; s < MAXF; s++) {
@@ -1100,7 +1127,7 @@ __global__ __launch_bounds__(BLOCK) void k_patch_rec(const FluxArgs<float> fa, c
         }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < npf; i += BLOCK) {
+    for (int i = threadIdx.x; i < npf; i += NT) {
         int64_t f;
         int info;
         patch_face(p, fa.finfo, f0 + i, f, info);
@@ -1125,10 +1152,11 @@ __global__ __launch_bounds__(BLOCK) void k_patch_rec(const FluxArgs<float> fa, c
 #pragma unroll
         for (int k = 0; k < NV; k++) L.g[k * npf + i] = g[k];
     }
+    const double dt = stage_dt(a);
     __syncthreads();
     double r[NV];
     patch_sum<NV, MAXF, true>(L.g, npf, cl, r);
-    stage_tail<NV, true, true>(a, c, valid, r, blk, a.l2, a.dtred);
+    stage_tail<NV, true, true, NT>(a, c, valid, dt, r, blk, a.l2, a.dtred);
 }
 
 // Resident waves per SIMD requested for the fused kernel, where the bound costs no more than a register
@@ -1143,14 +1171,15 @@ constexpr int fused_waves() {
     return ((SCHEME == MST_SCHEME_ROE || LIM == MST_LIM_NONE) && MAXF == 3) ? 4 : 1;
 }
 
-// Phases of one patch in the fused form, for a block of BLOCK lanes: the limited gradients of the
+// Phases of one patch in the fused form, for a block of NT lanes: the limited gradients of the
 // patch cells [cb, ce) and of the patch's halo, their face states into LDS, then the fluxes of the
 // patch faces (p.face from f0) into L.g.  Ends with a barrier.  cl receives the lane's cell's slot
 // entries ((local face << 1) | side, -1: none) for the caller's sums.  roe picks the scheme when
 // SCHEME is SCHEME_RUNTIME.  pre() runs between the gradient and the flux phases, when the gradient's
 // registers are free: the caller fetches its update's inputs there, so their latency overlaps the
-// face solves.
-template <int DIM, int SCHEME, int LIM, typename T, int MAXF, bool NRM_LDS = false, typename Pre>
+// face solves.  NT = 2 BLOCK: the lanes past the patch's cells take the halo's gradients at the same time, and
+// the patch's faces take one pass.
+template <int DIM, int SCHEME, int LIM, typename T, int MAXF, bool NRM_LDS = false, int NT = BLOCK, typename Pre>
 __device__ __forceinline__ void fused_patch(const GradArgs<T> &ga, const FluxArgs<T> &fa, bool roe, const PatchArgs &p,
                                             const HaloArgs &h, int64_t patch, int64_t cb, int64_t ce, int64_t nc,
                                             int32_t f0, FusedLds<T> &L, int (&cl)[MAXF], Pre pre) {
@@ -1159,13 +1188,13 @@ __device__ __forceinline__ void fused_patch(const GradArgs<T> &ga, const FluxArg
     // Inputs of the later phases that do not depend on the gradients are fetched first, so their
     // latency overlaps the gradient phase: each lane's first PF patch faces (face, kind, normal), its
     // cell's slot entries and its first halo cell.
-    constexpr int PF = MST_FUSED_PF;
+    constexpr int PF = NT > BLOCK ? 1 : MST_FUSED_PF;
     int64_t pf_f[PF];
     int pf_info[PF];
     double pf_n[PF][DIM];
 #pragma unroll
     for (int q = 0; q < PF; q++) {
-        const int i = threadIdx.x + q * BLOCK;
+        const int i = threadIdx.x + q * NT;
         pf_f[q] = -1;
         pf_info[q] = 0;
         if (i < npf) {
@@ -1175,12 +1204,15 @@ __device__ __forceinline__ void fused_patch(const GradArgs<T> &ga, const FluxArg
         }
     }
     const int64_t c = cb + threadIdx.x;
+    const bool mine = (NT == BLOCK || threadIdx.x < BLOCK) && c < ce;
 #pragma unroll
-    for (int s = 0; s < MAXF; s++) cl[s] = c < ce ? p.loc[(int64_t)s * nc + c] : -1;
+    for (int s = 0; s < MAXF; s++) cl[s] = mine ? p.loc[(int64_t)s * nc + c] : -1;
     // limited gradients of the patch cells, then of the halo cells; face states into LDS
     const int32_t h0 = h.start[patch];
-    const int next = BLOCK + (h.start[patch + 1] - h0);
-    const int32_t hc = BLOCK + (int)threadIdx.x < next ? h.cell[h0 + threadIdx.x] : 0;  // first halo pass
+    const int next = BLOCK + (h.start[patch + 1] - h0);  // the patch's cells, then its halo
+    // the lane's first halo cell (a wide block: of the lanes past the patch's cells)
+    const int j0 = NT > BLOCK ? (int)threadIdx.x - BLOCK : (int)threadIdx.x;
+    const int32_t hc = (NT == BLOCK || j0 >= 0) && BLOCK + j0 < next ? h.cell[h0 + j0] : 0;
     const IncView<T> own = cell_view(ga);
     const IncView<T> hv{h.code, static_cast<const T *>(h.w), static_cast<const T *>(h.n),
                         static_cast<const T *>(h.dx), static_cast<const GradVol<T> *>(h.vol), h.nh};
@@ -1191,16 +1223,15 @@ __device__ __forceinline__ void fused_patch(const GradArgs<T> &ga, const FluxArg
         // (not a patch face) reads the incidence array.
         GradIn<DIM, MAXF, T> gin;
         T dxs[MAXF][DIM];
-        const bool mine = c < ce;
         if (mine) grad_fetch<DIM, MAXF, false, T>(ga.Q, own, c, c, gin, dxs);
 #pragma unroll
         for (int q = 0; q < PF; q++) {
-            const int i = threadIdx.x + q * BLOCK;
+            const int i = threadIdx.x + q * NT;
             if (i < npf)
 #pragma unroll
                 for (int d = 0; d < DIM; d++) L.nrm[d * npf + i] = pf_n[q][d];
         }
-        for (int i = threadIdx.x + PF * BLOCK; i < npf; i += BLOCK) {
+        for (int i = threadIdx.x + PF * NT; i < npf; i += NT) {
             const int64_t f = p.face[f0 + i];
 #pragma unroll
             for (int d = 0; d < DIM; d++) L.nrm[d * npf + i] = fa.fn[f * DIM + d];
@@ -1237,13 +1268,15 @@ __device__ __forceinline__ void fused_patch(const GradArgs<T> &ga, const FluxArg
             }
         }
     }
-    for (int i0 = NRM_LDS ? BLOCK : 0; i0 < next; i0 += BLOCK) {  // i0 == 0: the patch cells, then the halo
+    for (int i0 = NRM_LDS && NT == BLOCK ? BLOCK : 0; i0 < next; i0 += NT) {
         const int i = i0 + (int)threadIdx.x;
         if (i >= next) break;
+        if (NRM_LDS && NT > BLOCK && i < BLOCK) continue;  // done above
         int64_t cc, g;
         const int16_t *lp;
         int64_t stride;
-        if (i0 == 0) {
+        const bool halo = NT == BLOCK ? i0 > 0 : i >= BLOCK;
+        if (!halo) {
             cc = cb + i;
             if (cc >= ce) continue;
             g = cc;
@@ -1256,7 +1289,7 @@ __device__ __forceinline__ void fused_patch(const GradArgs<T> &ga, const FluxArg
             stride = 1;
         }
         T qc[NV], lgr[NV * DIM], dxs[MAXF][DIM], t[NV][DIM], ph[NV];
-        const int nfc = grad_limited<DIM, MAXF, LIM, T>(ga.Q, i0 == 0 ? own : hv, g, cc, qc, lgr, dxs, t, ph);
+        const int nfc = grad_limited<DIM, MAXF, LIM, T>(ga.Q, halo ? hv : own, g, cc, qc, lgr, dxs, t, ph);
 #pragma unroll
         for (int s = 0; s < MAXF; s++) {
             if (s >= nfc) break;
@@ -1274,7 +1307,7 @@ __device__ __forceinline__ void fused_patch(const GradArgs<T> &ga, const FluxArg
     pre();
     // the patch's face fluxes (face_load's inputs from LDS: both sides' states, or for a boundary
     // face the raw interior state from memory and its reconstructed state)
-    for (int q = 0, i = threadIdx.x; i < npf; q++, i += BLOCK) {
+    for (int q = 0, i = threadIdx.x; i < npf; q++, i += NT) {
         int64_t f;
         int info;
         double n64[DIM];
@@ -1315,8 +1348,8 @@ __device__ __forceinline__ void fused_patch(const GradArgs<T> &ga, const FluxArg
     __syncthreads();
 }
 
-template <int DIM, int SCHEME, int LIM, typename T, int MAXF>
-__global__ __launch_bounds__(BLOCK, (fused_waves<DIM, SCHEME, LIM, T, MAXF>())) void k_fused(
+template <int DIM, int SCHEME, int LIM, typename T, int MAXF, int NT = BLOCK>
+__global__ __launch_bounds__(NT, (NT > BLOCK ? 2 : fused_waves<DIM, SCHEME, LIM, T, MAXF>())) void k_fused(
     const GradArgs<T> ga, const FluxArgs<T> fa, const UpdArgs a, const PatchArgs p, const HaloArgs h) {
     constexpr int NV = DIM + 2;
     constexpr bool F32 = std::is_same<T, float>::value;
@@ -1327,15 +1360,18 @@ __global__ __launch_bounds__(BLOCK, (fused_waves<DIM, SCHEME, LIM, T, MAXF>())) 
     const int64_t cb = blk * BLOCK, ce = cb + BLOCK < a.nc ? cb + BLOCK : a.nc;
     int cl[MAXF];
     const int64_t c = cb + threadIdx.x;
-    const bool valid = c < a.nc;
+    const bool valid = (NT == BLOCK || threadIdx.x < BLOCK) && c < a.nc;
     StageIn<NV> in;
-    fused_patch<DIM, SCHEME, LIM, T, MAXF, fused_lds_normals<DIM>()>(ga, fa, SCHEME == MST_SCHEME_ROE, p, h, blk, cb, ce,
-                                                                      a.nc, f0, L, cl, [&]() {
+    double dt = 0;
+    fused_patch<DIM, SCHEME, LIM, T, MAXF, fused_lds_normals<DIM>(), NT>(ga, fa, SCHEME == MST_SCHEME_ROE, p, h, blk, cb,
+                                                                          ce, a.nc, f0, L, cl, [&]() {
+        dt = stage_dt(a);
         if (valid) stage_load<NV, F32>(a, c, in);
     });
     double r[NV];
     patch_sum<NV, MAXF, F32>(L.g, L.npf, cl, r);
-    stage_tail<NV, true, F32, true>(a, c, valid, r, blk, a.l2, a.dtred, &in, sh);  // (sh at least NV * BLOCK / 64 doubles)
+    // (sh: at least NV * NT / 64 doubles)
+    stage_tail<NV, true, F32, NT, true>(a, c, valid, dt, r, blk, a.l2, a.dtred, &in, sh);
 }
 
 // ------------------------------------------------------------------------------------ reductions

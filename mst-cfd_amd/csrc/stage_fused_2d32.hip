@@ -1,0 +1,6 @@
+// Fused strategy, 2D, the mixed form.
+#include "stage_fused.hpp"
+
+namespace mstk {
+template int run_fused_t<2, float>(mst_ctx *, int, int, int, const Stage &, int);
+}

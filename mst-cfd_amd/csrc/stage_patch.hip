@@ -1,0 +1,84 @@
+// stage_patch.hip -- launches of the patch strategy.
+#include "context.hpp"
+
+namespace mstk {
+
+// patch strategy: gradient + limiter (order 2), then the patch kernel (faces into LDS, sum, update)
+template <int DIM, typename T>
+int run_patch_t(mst_ctx *x, int mode, int is, int in, const Stage &sg, int iout) {
+    if (!x->patch_ok) return mst::fail(MST_E_UNSUPPORTED, "no patch tables for this mesh");
+    const FluxArgs<T> fa = flux_args<T>(x, is);
+    const UpdArgs a = upd_args(x, mode, is, in, sg, iout);
+    PatchArgs pa;
+    pa.start = x->pstart;
+    pa.face = x->pface;
+    pa.loc = x->ploc;
+    pa.fi = x->pfi;
+    const size_t shm = (size_t)x->max_pf * x->nv * sizeof(double);
+    const bool second = x->cfg.order >= 2;
+    const bool roe = x->cfg.scheme == MST_SCHEME_ROE;
+    if constexpr (std::is_same<T, float>::value) {
+        if (second) {  // the mixed form stages its face states in LDS from the records (k_patch_rec)
+            HaloArgs ha{};
+            ha.start = x->hstart;
+            ha.cell = x->hcell;
+            ha.loc = x->hloc;
+#define MST_PATCH_REC_N(MF, NT)                                                                                     \
+    return roe ? launch_nt(x, MST_K_PATCH, k_patch_rec<DIM, MST_SCHEME_ROE, MF, NT>, x->nc, NT, shm, fa, a, pa, ha) \
+               : launch_nt(x, MST_K_PATCH, k_patch_rec<DIM, MST_SCHEME_AUSM, MF, NT>, x->nc, NT, shm, fa, a, pa, ha);
+#define MST_PATCH_REC(MF)                       \
+    if (x->wide_patch) { MST_PATCH_REC_N(MF, 2 * BLOCK) } \
+    MST_PATCH_REC_N(MF, BLOCK)
+            if (x->slots == 3) { MST_PATCH_REC(3) }
+            MST_PATCH_REC(4)
+#undef MST_PATCH_REC
+#undef MST_PATCH_REC_N
+        }
+    }
+#define MST_PATCH_N(MF, SECOND, NT)                                                                                       \
+    return roe ? launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_ROE, SECOND, T, MF, true, NT>, x->nc, NT, shm, fa, a, pa) \
+               : launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_AUSM, SECOND, T, MF, true, NT>, x->nc, NT, shm, fa, a, pa);
+#define MST_PATCH(MF)                                    \
+    if (x->wide_patch) {                                       \
+        if (second) { MST_PATCH_N(MF, true, 2 * BLOCK) } \
+        MST_PATCH_N(MF, false, 2 * BLOCK)                \
+    }                                                    \
+    if (second) { MST_PATCH_N(MF, true, BLOCK) }         \
+    MST_PATCH_N(MF, false, BLOCK)
+    if (x->slots == 3) { MST_PATCH(3) }
+    MST_PATCH(4)
+#undef MST_PATCH
+#undef MST_PATCH_N
+}
+
+template <int DIM>
+int run_patch_residual_t(mst_ctx *x, int mode, int is) {
+    const FluxArgs<double> fa = flux_args<double>(x, is);
+    const UpdArgs a = upd_args(x, mode, is, -1, Stage{0, 0}, -1);
+    PatchArgs pa;
+    pa.start = x->pstart;
+    pa.face = x->pface;
+    pa.loc = x->ploc;
+    pa.fi = x->pfi;
+    const size_t shm = (size_t)x->max_pf * x->nv * sizeof(double);
+    const bool second = x->cfg.order >= 2;
+    const bool roe = x->cfg.scheme == MST_SCHEME_ROE;
+#define MST_PATCH_R(MF)                                                                                          \
+    if (roe)                                                                                                     \
+        return second ? launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_ROE, true, double, MF, false>, x->nc, BLOCK, shm, fa, a, pa) \
+                      : launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_ROE, false, double, MF, false>, x->nc, BLOCK, shm, fa, a, pa); \
+    return second ? launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_AUSM, true, double, MF, false>, x->nc, BLOCK, shm, fa, a, pa)    \
+                  : launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_AUSM, false, double, MF, false>, x->nc, BLOCK, shm, fa, a, pa);
+    if (x->slots == 3) { MST_PATCH_R(3) }
+    MST_PATCH_R(4)
+#undef MST_PATCH_R
+}
+
+template int run_patch_t<2, double>(mst_ctx *, int, int, int, const Stage &, int);
+template int run_patch_t<3, double>(mst_ctx *, int, int, int, const Stage &, int);
+template int run_patch_t<2, float>(mst_ctx *, int, int, int, const Stage &, int);
+template int run_patch_t<3, float>(mst_ctx *, int, int, int, const Stage &, int);
+template int run_patch_residual_t<2>(mst_ctx *, int, int);
+template int run_patch_residual_t<3>(mst_ctx *, int, int);
+
+}  // namespace mstk
