@@ -14,6 +14,7 @@
 #include "mstcfd.h"
 #include "prep.hpp"
 #include "transfer.hpp"
+#include "viscous.hpp"
 
 using namespace mstk;
 
@@ -86,7 +87,8 @@ struct mst_ctx {
     int *bad = nullptr;
     int32_t *cnew = nullptr;  // device position of each file cell
     Transfer link;            // host states in file order
-    bool viscous = false;     // mu or kappa > 0: the face strategy with the viscous kernels
+    bool viscous = false;     // mu or kappa > 0: the viscous kernels (viscous.hpp), patch or face route
+    bool visc_patch = false;  // the mesh allows the patch route
     double *gw = nullptr;     // viscous: per cell Green-Gauss gradients of (u, T), [nc][dim + 1][dim]
     // LU-SGS steady driver (built on first use): cell colours, the cells of each colour in ascending
     // order (colour k: lu_cells[lu_start[k] .. lu_start[k + 1])), face spectral radii, the update
@@ -223,10 +225,35 @@ inline UpdArgs upd_args(const mst_ctx *x, int mode, int is, int in, const Stage 
     return a;
 }
 
+inline ViscArgs visc_args(const mst_ctx *x, int isrc) {
+    ViscArgs a;
+    a.nc = x->nc;
+    a.nf = x->nf;
+    a.inc_code = x->inc_code;
+    a.ell = x->ell;
+    a.finfo = x->finfo;
+    a.inc_w = x->inc_w;
+    a.inc_n = x->inc_n;
+    a.vol = x->cvol;
+    a.fc0 = x->fc0;
+    a.fc1 = x->fc1;
+    a.feta = x->feta;
+    a.fn = x->fn;
+    a.Q = x->Q[isrc];
+    a.gw = x->gw;
+    a.G = x->G;
+    a.mu = x->cfg.mu;
+    a.lam = x->cfg.lam;
+    a.kappa = x->cfg.kappa;
+    a.cv = x->cfg.cv;
+    return a;
+}
+
 // one stage (mode includes UPD_STAGE) with the patch strategy (its gradient kernel has run) or the fused one;
 // explicitly instantiated in their files
 template <int DIM, typename T>
 int run_patch_t(mst_ctx *x, int mode, int is, int in, const Stage &sg, int iout);
+// (a viscous configuration: its viscous gradients have run too)
 template <int DIM, typename T>
 int run_fused_t(mst_ctx *x, int mode, int is, int in, const Stage &sg, int iout);
 // the patch kernel's residual-only form (FP64): R of state is, and its L2 partials when mode has UPD_L2

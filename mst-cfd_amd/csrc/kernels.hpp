@@ -394,14 +394,12 @@ __device__ __forceinline__ IncView<T> cell_view(const GradArgs<T> &a) {
     return IncView<T>{a.inc_code, a.inc_w, a.inc_n, a.inc_dx, a.vol, a.nc};
 }
 
-// grad_limited, then the cell's face records and the optional raw gradient / limiter outputs
-template <int DIM, int MAXF, int LIM, typename T>
-__device__ __forceinline__ void grad_cell(const GradArgs<T> &a, const int64_t c) {
+// reconstructed states at the cell's faces (RhoSolver.cpp:250,254 with the limiter), one record per
+// incidence, coalesced over the cells of a slot
+template <int DIM, int MAXF, typename T>
+__device__ __forceinline__ void grad_records(const GradArgs<T> &a, const int64_t c, int nfc, const T (&qc)[DIM + 2],
+                                             const T (&lgr)[(DIM + 2) * DIM], const T (&dxs)[MAXF][DIM]) {
     constexpr int NV = DIM + 2;
-    T qc[NV], lgr[NV * DIM], dxs[MAXF][DIM], t[NV][DIM], ph[NV];
-    const int nfc = grad_limited<DIM, MAXF, LIM, T>(a.Q, cell_view(a), c, c, qc, lgr, dxs, t, ph);
-    // reconstructed states at the cell's faces (RhoSolver.cpp:250,254 with the limiter), one record
-    // per incidence, coalesced over the cells of a slot
 #pragma unroll
     for (int s = 0; s < MAXF; s++) {
         if (s >= nfc) break;
@@ -411,6 +409,15 @@ __device__ __forceinline__ void grad_cell(const GradArgs<T> &a, const int64_t c)
         recon<DIM>(q, lgr, dxs[s]);
         stq<NV>(a.rec + ((int64_t)s * a.nc + c) * NV, q);
     }
+}
+
+// grad_limited, then the cell's face records and the optional raw gradient / limiter outputs
+template <int DIM, int MAXF, int LIM, typename T>
+__device__ __forceinline__ void grad_cell(const GradArgs<T> &a, const int64_t c) {
+    constexpr int NV = DIM + 2;
+    T qc[NV], lgr[NV * DIM], dxs[MAXF][DIM], t[NV][DIM], ph[NV];
+    const int nfc = grad_limited<DIM, MAXF, LIM, T>(a.Q, cell_view(a), c, c, qc, lgr, dxs, t, ph);
+    grad_records<DIM, MAXF, T>(a, c, nfc, qc, lgr, dxs);
     if (a.graw) {
 #pragma unroll
         for (int k = 0; k < NV; k++)
@@ -909,9 +916,15 @@ __device__ __forceinline__ void patch_sum(const double *g, int npf, const int (&
 }
 
 // STAGE false: the residual only (R and, with a.l2, its norms), for the implicit steady driver.  NT lanes per patch of
-// BLOCK cells: twice as many on meshes of few patches, where the patch's faces then take one pass.
-template <int DIM, int SCHEME, bool SECOND, typename T, int MAXF, bool STAGE = true, int NT = BLOCK>
-__global__ __launch_bounds__(NT) void k_patch(const FluxArgs<T> fa, const UpdArgs a, const PatchArgs p) {
+// BLOCK cells: twice as many on meshes of few patches, where the patch's faces then take one pass.  extra: what is
+// added to a face's flux (the viscous terms).
+struct NoExtra {
+    template <typename G>
+    __device__ __forceinline__ void operator()(int64_t, int, G &) const {}
+};
+template <int DIM, int SCHEME, bool SECOND, typename T, int MAXF, bool STAGE = true, int NT = BLOCK, typename Extra = NoExtra>
+__global__ __launch_bounds__(NT) void k_patch(const FluxArgs<T> fa, const UpdArgs a, const PatchArgs p,
+                                              const Extra extra = Extra()) {
     constexpr int NV = DIM + 2;
     constexpr bool F32 = std::is_same<T, float>::value;
     extern __shared__ double gsh[];  // NV x npf, component-major: consecutive lanes, consecutive banks
@@ -924,6 +937,7 @@ __global__ __launch_bounds__(NT) void k_patch(const FluxArgs<T> fa, const UpdArg
         patch_face(p, fa.finfo, f0 + i, f, info);
         double g[NV];
         face_flux<DIM, SCHEME, SECOND, T>(fa, f, info & 15, info >> 4, g);
+        extra(f, info & 15, g);
 #pragma unroll
         for (int k = 0; k < NV; k++) gsh[k * npf + i] = g[k];
     }

@@ -84,38 +84,43 @@ int run_flux_t(mst_ctx *x, int isrc) {
                   : launch(x, MST_K_FLUX, k_flux<DIM, MST_SCHEME_AUSM, false, T>, x->nf, a);
 }
 
+// viscous gradients of the cells of state isrc
+int run_visc_grad(mst_ctx *x, int isrc) {
+    const ViscArgs a = visc_args(x, isrc);
+    if (x->dim == 2)
+        return x->slots == 3 ? launch(x, MST_K_VISC, k_visc_grad<2, 3>, x->nc, a)
+                             : (x->slots == 4 ? launch(x, MST_K_VISC, k_visc_grad<2, 4>, x->nc, a)
+                                              : launch(x, MST_K_VISC, k_visc_grad<2, 8>, x->nc, a));
+    return x->slots == 4 ? launch(x, MST_K_VISC, k_visc_grad<3, 4>, x->nc, a)
+                         : launch(x, MST_K_VISC, k_visc_grad<3, 8>, x->nc, a);
+}
+
 // viscous terms of state isrc subtracted from the face fluxes (after the flux kernel)
 int run_viscous(mst_ctx *x, int isrc) {
-    ViscArgs a;
-    a.nc = x->nc;
-    a.nf = x->nf;
-    a.inc_code = x->inc_code;
-    a.ell = x->ell;
-    a.finfo = x->finfo;
-    a.inc_w = x->inc_w;
-    a.inc_n = x->inc_n;
-    a.vol = x->cvol;
-    a.fc0 = x->fc0;
-    a.fc1 = x->fc1;
-    a.feta = x->feta;
-    a.fn = x->fn;
-    a.Q = x->Q[isrc];
-    a.gw = x->gw;
-    a.G = x->G;
-    a.mu = x->cfg.mu;
-    a.lam = x->cfg.lam;
-    a.kappa = x->cfg.kappa;
-    a.cv = x->cfg.cv;
-    int rc;
-    if (x->dim == 2)
-        rc = x->slots == 3 ? launch(x, MST_K_VISC, k_visc_grad<2, 3>, x->nc, a)
-                           : (x->slots == 4 ? launch(x, MST_K_VISC, k_visc_grad<2, 4>, x->nc, a)
-                                            : launch(x, MST_K_VISC, k_visc_grad<2, 8>, x->nc, a));
-    else
-        rc = x->slots == 4 ? launch(x, MST_K_VISC, k_visc_grad<3, 4>, x->nc, a)
-                           : launch(x, MST_K_VISC, k_visc_grad<3, 8>, x->nc, a);
+    const int rc = run_visc_grad(x, isrc);
     if (rc) return rc;
+    const ViscArgs a = visc_args(x, isrc);
     return x->dim == 2 ? launch(x, MST_K_VISC, k_visc_flux<2>, x->nf, a) : launch(x, MST_K_VISC, k_visc_flux<3>, x->nf, a);
+}
+
+// gradients of a viscous stage on the patch route: face states and viscous gradients in one kernel (order 2, FP64)
+template <int DIM, int MF>
+int run_grad_visc_t(mst_ctx *x, int isrc) {
+    const GradArgs<double> g = grad_args<double>(x, isrc, false);
+    const ViscArgs v = visc_args(x, isrc);
+    if (x->cfg.limiter == MST_LIM_NONE) return launch(x, MST_K_GRAD, k_grad_visc<DIM, MF, MST_LIM_NONE>, x->nc, g, v);
+    if (x->cfg.limiter == MST_LIM_MINMOD) return launch(x, MST_K_GRAD, k_grad_visc<DIM, MF, MST_LIM_MINMOD>, x->nc, g, v);
+    return launch(x, MST_K_GRAD, k_grad_visc<DIM, MF, MST_LIM_VANLEER>, x->nc, g, v);
+}
+
+int run_grad_visc(mst_ctx *x, int isrc) {
+    if (x->cfg.order >= 2 && !x->mixed) {
+        if (x->dim == 2) return x->slots == 3 ? run_grad_visc_t<2, 3>(x, isrc) : run_grad_visc_t<2, 4>(x, isrc);
+        return run_grad_visc_t<3, 4>(x, isrc);
+    }
+    int rc = MST_OK;
+    if (x->cfg.order >= 2) rc = run_grad(x, isrc, false);
+    return rc ? rc : run_visc_grad(x, isrc);
 }
 
 // residual evaluation up to the face fluxes: gradient + limiter (order 2), the flux kernel, and the
@@ -194,13 +199,25 @@ int run_stage(mst_ctx *x, int mode, int is, int in, const Stage &sg, int iout) {
         int rc = resolve_strategy(x);
         if (rc) return rc;
     }
-    if (x->resolved == MST_STRATEGY_FACE || x->viscous) {  // the viscous kernels follow the flux kernel
+    if (x->resolved == MST_STRATEGY_FACE || (x->viscous && !x->visc_patch)) {
         int rc = run_face_flux(x, is);
         if (rc) return rc;
         return run_update(x, mode, is, in, sg, iout);
     }
     int rc = ensure_shadow(x, is);
     if (rc) return rc;
+    if (x->viscous) {  // the patch route, whichever of the other strategies is set
+        rc = run_grad_visc(x, is);
+        if (rc) return rc;
+        if (x->mixed)
+            rc = x->dim == 2 ? run_patch_t<2, float>(x, mode, is, in, sg, iout)
+                             : run_patch_t<3, float>(x, mode, is, in, sg, iout);
+        else
+            rc = x->dim == 2 ? run_patch_t<2, double>(x, mode, is, in, sg, iout)
+                             : run_patch_t<3, double>(x, mode, is, in, sg, iout);
+        if (rc == MST_OK && iout >= 0) x->shadow_ok[iout] = x->mixed;
+        return rc;
+    }
     if (x->resolved == MST_STRATEGY_FUSED) {
         if (x->mixed)
             rc = x->dim == 2 ? run_fused_t<2, float>(x, mode, is, in, sg, iout)
@@ -503,6 +520,9 @@ int upload_config(mst_ctx *x) {
     x->p32 = make_params<float>(x->cfg);
     x->mixed = x->cfg.precision == MST_PREC_MIXED;
     x->viscous = x->cfg.mu > 0 || x->cfg.kappa > 0;
+    // (a face of unknown type is in no patch list, but its cell's viscous flux counts: the face route)
+    x->visc_patch = x->patch_ok && std::find(x->prep.P.fkind.begin(), x->prep.P.fkind.end(), (int32_t)mst::KIND_NONE) ==
+                                       x->prep.P.fkind.end();
     if (x->viscous && !x->gw) {
         int rc = dalloc(&x->gw, (size_t)(x->nc * (x->dim + 1) * x->dim));
         if (rc) return rc;
@@ -756,6 +776,8 @@ int resolve_strategy(mst_ctx *x) {
     for (int s : {MST_STRATEGY_FACE, MST_STRATEGY_CELL, MST_STRATEGY_PATCH, MST_STRATEGY_FUSED}) {
         if ((s == MST_STRATEGY_PATCH || s == MST_STRATEGY_FUSED) && !x->patch_ok) continue;
         if (s == MST_STRATEGY_FUSED && !x->fused_ok) continue;
+        // viscous stages have two routes: the face strategy's, and the patch route under any other
+        if (x->viscous && s != MST_STRATEGY_FACE && s != (x->patch_ok ? MST_STRATEGY_PATCH : MST_STRATEGY_CELL)) continue;
         x->resolved = s;
         rc = run_stage(x, UPD_STAGE, x->iold, x->iold, Stage{}, spare);  // warm-up
         if (rc) break;
@@ -1476,6 +1498,7 @@ int mst_algorithmic_bytes(const mst_ctx *ctx, int kernel, double *bytes) {
         case MST_K_GRAD:  // incidences: code, weight (not FP32 3D: folded into the normal), normal, offset,
                           // record out; cells: state, volume
             *bytes = 4.0 * ctx->slots * nc + ninc * (w_inc + 2 * r * D + r * NV) + nc * (r * NV + r);
+            if (ctx->viscous && ctx->visc_patch && !mixed) *bytes += nc * 8 * (D + 1) * D;  // viscous gradients out
             break;
         case MST_K_UPDATE:
             *bytes = upd + nf * 8 * NV;
@@ -1487,6 +1510,7 @@ int mst_algorithmic_bytes(const mst_ctx *ctx, int kernel, double *bytes) {
             // (a face's kind comes with its packed list entry when there is one)
             *bytes = flux_in + upd - (mixed ? 0 : (second ? nbnd : nc) * 8 * NV) - ell +
                      4.0 * (double)ctx->n_psolve + 2.0 * ctx->slots * nc - (ctx->pfi ? 4.0 * nf : 0.0);
+            if (ctx->viscous) *bytes += nc * 8 * ((D + 1) * D + (second ? NV : 0)) + nf * 16;  // viscous terms' inputs
             break;
         case MST_K_FUSED: {  // gradient inputs + per-face inputs + update, each once; no records
             // per incidence: code, weight, offset, and in 3D the normal (2D takes it from its face's)

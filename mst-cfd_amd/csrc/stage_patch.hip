@@ -17,6 +17,21 @@ int run_patch_t(mst_ctx *x, int mode, int is, int in, const Stage &sg, int iout)
     const size_t shm = (size_t)x->max_pf * x->nv * sizeof(double);
     const bool second = x->cfg.order >= 2;
     const bool roe = x->cfg.scheme == MST_SCHEME_ROE;
+    if (x->viscous) {
+        const ViscFace<DIM> vf{visc_args(x, is)};
+#define MST_PATCH_V(MF, SECOND)                                                                                             \
+    return roe ? launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_ROE, SECOND, T, MF, true, BLOCK, ViscFace<DIM>>, x->nc, \
+                           BLOCK, shm, fa, a, pa, vf)                                                                       \
+               : launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_AUSM, SECOND, T, MF, true, BLOCK, ViscFace<DIM>>, x->nc, \
+                           BLOCK, shm, fa, a, pa, vf);
+        if (x->slots == 3) {
+            if (second) { MST_PATCH_V(3, true) }
+            MST_PATCH_V(3, false)
+        }
+        if (second) { MST_PATCH_V(4, true) }
+        MST_PATCH_V(4, false)
+#undef MST_PATCH_V
+    }
     if constexpr (std::is_same<T, float>::value) {
         if (second) {  // the mixed form stages its face states in LDS from the records (k_patch_rec)
             HaloArgs ha{};
@@ -36,8 +51,8 @@ int run_patch_t(mst_ctx *x, int mode, int is, int in, const Stage &sg, int iout)
         }
     }
 #define MST_PATCH_N(MF, SECOND, NT)                                                                                       \
-    return roe ? launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_ROE, SECOND, T, MF, true, NT>, x->nc, NT, shm, fa, a, pa) \
-               : launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_AUSM, SECOND, T, MF, true, NT>, x->nc, NT, shm, fa, a, pa);
+    return roe ? launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_ROE, SECOND, T, MF, true, NT>, x->nc, NT, shm, fa, a, pa, NoExtra()) \
+               : launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_AUSM, SECOND, T, MF, true, NT>, x->nc, NT, shm, fa, a, pa, NoExtra());
 #define MST_PATCH(MF)                                    \
     if (x->wide_patch) {                                       \
         if (second) { MST_PATCH_N(MF, true, 2 * BLOCK) } \
@@ -65,10 +80,10 @@ int run_patch_residual_t(mst_ctx *x, int mode, int is) {
     const bool roe = x->cfg.scheme == MST_SCHEME_ROE;
 #define MST_PATCH_R(MF)                                                                                          \
     if (roe)                                                                                                     \
-        return second ? launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_ROE, true, double, MF, false>, x->nc, BLOCK, shm, fa, a, pa) \
-                      : launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_ROE, false, double, MF, false>, x->nc, BLOCK, shm, fa, a, pa); \
-    return second ? launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_AUSM, true, double, MF, false>, x->nc, BLOCK, shm, fa, a, pa)    \
-                  : launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_AUSM, false, double, MF, false>, x->nc, BLOCK, shm, fa, a, pa);
+        return second ? launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_ROE, true, double, MF, false>, x->nc, BLOCK, shm, fa, a, pa, NoExtra()) \
+                      : launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_ROE, false, double, MF, false>, x->nc, BLOCK, shm, fa, a, pa, NoExtra()); \
+    return second ? launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_AUSM, true, double, MF, false>, x->nc, BLOCK, shm, fa, a, pa, NoExtra())    \
+                  : launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_AUSM, false, double, MF, false>, x->nc, BLOCK, shm, fa, a, pa, NoExtra());
     if (x->slots == 3) { MST_PATCH_R(3) }
     MST_PATCH_R(4)
 #undef MST_PATCH_R
