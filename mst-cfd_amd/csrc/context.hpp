@@ -93,6 +93,7 @@ struct mst_ctx {
     // LU-SGS steady driver (built on first use): cell colours, the cells of each colour in ascending
     // order (colour k: lu_cells[lu_start[k] .. lu_start[k + 1])), face spectral radii, the update
     int32_t *lu_cells = nullptr, *lu_nb = nullptr, *lu_face = nullptr;
+    uint32_t *lu_info = nullptr;
     std::vector<int64_t> lu_start;
     std::vector<int32_t> lu_colour;  // per cell (host copy)
     double *lu_n = nullptr, *lu_r = nullptr, *lu_D = nullptr, *lu_dQ = nullptr;

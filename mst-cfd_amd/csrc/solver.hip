@@ -501,6 +501,15 @@ int upload_incidence_weights(mst_ctx *x, const std::vector<double> &eta) {
     return MST_OK;
 }
 
+// the LU-SGS sweeps' face words, from the current kinds and masks (nothing before the colours are built)
+int lu_finfo(mst_ctx *x) {
+    if (!x->lu_info) return MST_OK;
+    hipLaunchKernelGGL(k_lu_finfo<0>, dim3((uint32_t)((x->nc + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, x->stream, x->nc,
+                       x->slots, (const int32_t *)x->lu_face, (const int32_t *)x->finfo, x->lu_info);
+    HIPCHK(hipGetLastError());
+    return MST_OK;
+}
+
 int upload_config(mst_ctx *x) {
     std::vector<int32_t> mask;
     mst::lr_masks(x->prep.P, x->cfg.compat, mask);
@@ -513,6 +522,8 @@ int upload_config(mst_ctx *x) {
                            (const int32_t *)x->pface, (const int32_t *)x->finfo, x->pfi);
         HIPCHK(hipGetLastError());
     }
+    int rc = lu_finfo(x);
+    if (rc) return rc;
     std::vector<double> eta = x->prep.P.feta;
     if ((x->cfg.compat & MST_COMPAT_GRAD_LASTINT) && x->prep.P.quirk_face >= 0) eta[x->prep.P.quirk_face] = 1.0;
     HIPCHK(hipMemcpy(x->feta, eta.data(), sizeof(double) * x->nf, hipMemcpyHostToDevice));
@@ -524,11 +535,11 @@ int upload_config(mst_ctx *x) {
     x->visc_patch = x->patch_ok && std::find(x->prep.P.fkind.begin(), x->prep.P.fkind.end(), (int32_t)mst::KIND_NONE) ==
                                        x->prep.P.fkind.end();
     if (x->viscous && !x->gw) {
-        int rc = dalloc(&x->gw, (size_t)(x->nc * (x->dim + 1) * x->dim));
+        rc = dalloc(&x->gw, (size_t)(x->nc * (x->dim + 1) * x->dim));
         if (rc) return rc;
     }
     if (x->mixed) {
-        int rc = alloc_mixed(x);
+        rc = alloc_mixed(x);
         if (rc) return rc;
         for (int i = 0; i < 4; i++) x->shadow_ok[i] = false;
     }
@@ -542,7 +553,7 @@ void release(mst_ctx *x) {
                     x->scal, x->part, x->fin_mid, x->bad, x->Q32[0], x->Q32[1], x->Q32[2], x->Q32[3], x->rec32,
                     x->frec0, x->frec1, x->inc_code, x->inc_w, x->inc_n, x->inc_dx, x->inc_w32, x->inc_n32,
                     x->inc_dx32, x->ivol32, x->pstart, x->pface, x->pfi, x->ploc, x->hstart, x->hcell, x->hloc,
-                    x->lu_cells, x->lu_nb, x->lu_face, x->lu_n, x->lu_r, x->lu_D, x->lu_dQ, x->gw, x->cnew, x->pdt[0], x->pdt[1]};
+                    x->lu_cells, x->lu_nb, x->lu_face, x->lu_info, x->lu_n, x->lu_r, x->lu_D, x->lu_dQ, x->gw, x->cnew, x->pdt[0], x->pdt[1]};
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     x->hg.release();
@@ -615,10 +626,17 @@ int build_colours(mst_ctx *x) {
     if (rc == MST_OK) rc = dalloc(&x->lu_D, (size_t)nc);
     if (rc == MST_OK) rc = dalloc(&x->lu_dQ, (size_t)(nc * x->nv));
     if (rc == MST_OK && !x->R) rc = dalloc(&x->R, (size_t)(nc * x->nv));
+    if (rc == MST_OK) rc = dalloc(&x->lu_info, (size_t)nc);
+    if (rc == MST_OK) rc = lu_finfo(x);
     if (rc) return rc;
     x->lu_start = start;
     x->lu_colour = std::move(col);
     return MST_OK;
+}
+
+template <typename K>
+int launch_lu(mst_ctx *x, K kernel, const LuArgs &a, int64_t t0, int64_t n) {
+    return launch_nt(x, MST_K_LUSGS, kernel, (n + LU_BLOCK - 1) / LU_BLOCK * BLOCK, LU_BLOCK, 0, a, t0, n);
 }
 
 // forward launches; RS >= 0: the first-order residual computed by the sweep (scheme RS)
@@ -628,8 +646,8 @@ int lu_forward(mst_ctx *x, const LuArgs &a) {
     int rc = MST_OK;
     for (int k = 0; k < ncol && rc == MST_OK; k++) {
         const int64_t t0 = x->lu_start[k], n = x->lu_start[k + 1] - t0;
-        rc = k == ncol - 1 ? launch(x, MST_K_LUSGS, k_lu_sweep<DIM, true, true, MAXF, RS>, n, a, t0, n)
-                           : launch(x, MST_K_LUSGS, k_lu_sweep<DIM, true, false, MAXF, RS>, n, a, t0, n);
+        rc = k == ncol - 1 ? launch_lu(x, k_lu_sweep<DIM, true, true, MAXF, RS>, a, t0, n)
+                           : launch_lu(x, k_lu_sweep<DIM, true, false, MAXF, RS>, a, t0, n);
     }
     return rc;
 }
@@ -649,7 +667,7 @@ int lu_sweeps(mst_ctx *x, const LuArgs &a, bool inline_res) {
     }
     for (int k = ncol - 2; k >= 0 && rc == MST_OK; k--) {
         const int64_t t0 = x->lu_start[k], n = x->lu_start[k + 1] - t0;
-        rc = launch(x, MST_K_LUSGS, k_lu_sweep<DIM, false, false, MAXF>, n, a, t0, n);
+        rc = launch_lu(x, k_lu_sweep<DIM, false, false, MAXF>, a, t0, n);
     }
     return rc;
 }
@@ -672,8 +690,7 @@ LuArgs lu_args(const mst_ctx *x) {
     a.gamma = x->cfg.gamma;
     a.omega = x->lu_omega;
     a.dscale = 1.0 / x->lu_cfl + 0.5 * x->lu_omega;
-    a.face = x->lu_face;
-    a.finfo = x->finfo;
+    a.finfo = x->lu_info;
     a.P = x->p64;
     return a;
 }
@@ -729,16 +746,16 @@ int lu_inline_run(mst_ctx *x, int n) {
         const LuArgs a = lu_args(x);
         for (int k = it == 0 ? 0 : 1; k < ncol && rc == MST_OK; k++) {  // colour 0: done by the fused launch
             const int64_t t0 = x->lu_start[k], m = x->lu_start[k + 1] - t0;
-            rc = k == ncol - 1 ? launch(x, MST_K_LUSGS, k_lu_sweep<DIM, true, true, MAXF, RS>, m, a, t0, m)
-                               : launch(x, MST_K_LUSGS, k_lu_sweep<DIM, true, false, MAXF, RS>, m, a, t0, m);
+            rc = k == ncol - 1 ? launch_lu(x, k_lu_sweep<DIM, true, true, MAXF, RS>, a, t0, m)
+                               : launch_lu(x, k_lu_sweep<DIM, true, false, MAXF, RS>, a, t0, m);
         }
         for (int k = ncol - 2; k >= 1 && rc == MST_OK; k--) {
             const int64_t t0 = x->lu_start[k], m = x->lu_start[k + 1] - t0;
-            rc = launch(x, MST_K_LUSGS, k_lu_sweep<DIM, false, false, MAXF>, m, a, t0, m);
+            rc = launch_lu(x, k_lu_sweep<DIM, false, false, MAXF>, a, t0, m);
         }
         if (rc) break;
-        rc = it < n - 1 ? launch(x, MST_K_LUSGS, k_lu_sweep_bf<DIM, MAXF, RS>, n0, a, x->lu_start[0], n0)
-                        : launch(x, MST_K_LUSGS, k_lu_sweep<DIM, false, false, MAXF>, n0, a, x->lu_start[0], n0);
+        rc = it < n - 1 ? launch_lu(x, k_lu_sweep_bf<DIM, MAXF, RS>, a, x->lu_start[0], n0)
+                        : launch_lu(x, k_lu_sweep<DIM, false, false, MAXF>, a, x->lu_start[0], n0);
         x->shadow_ok[x->inew] = false;
         std::swap(x->iold, x->inew);
     }
