@@ -71,7 +71,7 @@ struct mst_ctx {
     double *inc_w = nullptr, *inc_n = nullptr, *inc_dx = nullptr;
     float *inc_w32 = nullptr, *inc_n32 = nullptr, *inc_dx32 = nullptr;
     float *ivol32 = nullptr;  // (float) 1/V, the FP32 gradient's volume input
-    double *scal = nullptr;  // [0] dt, [1..5] l2 norms, [6..10] maxrel
+    double *scal = nullptr;  // [0] dt, [1..5] l2 norms
     double *part = nullptr;  // per-block partials
     double *fin_mid = nullptr;  // first-level results of the two-level finish
     bool dt_valid = false;   // scal[0] holds the CFL time step of the current Old state
@@ -85,6 +85,8 @@ struct mst_ctx {
     // 36 / 32 (41), 57.0 / 54.4 (324), 80.3 / 80.9 (633).
     bool wide_patch = false, wide_fused = false;
     int *bad = nullptr;
+    Board *board = nullptr;  // pinned: the words the host waits for
+    uint32_t board_seq = 0;
     int32_t *cnew = nullptr;  // device position of each file cell
     Transfer link;            // host states in file order
     bool viscous = false;     // mu or kappa > 0: the viscous kernels (viscous.hpp), patch or face route

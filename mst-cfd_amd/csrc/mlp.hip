@@ -1127,18 +1127,32 @@ double sum_host(const float *dptr, int64_t n) {
 
 namespace mst {
 
+// later work of stream `after` waits for the earlier work of `before` (an event of its own per call: threads may share
+// a network)
+static int follow(hipStream_t after, hipStream_t before) {
+    if (after == before) return MST_OK;
+    hipEvent_t ev = nullptr;
+    HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    hipError_t e = hipEventRecord(ev, before);
+    if (e == hipSuccess) e = hipStreamWaitEvent(after, ev, 0);
+    (void)hipEventDestroy(ev);
+    HIPCHK(e);
+    return MST_OK;
+}
+
 int mlp_forward_device(mst_mlp *q, const float *dX, int64_t rows, float *dY, hipStream_t stream) {
     if (use_net(q)) {
         int rc = ensure_pack(q);
         if (rc) return rc;
-        HIPCHK(hipStreamSynchronize(stream));  // the inputs (the network runs on its own stream)
+        // the network runs on its own stream, between the caller's earlier and later work
+        rc = follow(q->stream, stream);
+        if (rc) return rc;
         NetArgs a = net_args(q, rows);
         a.X = dX;
         a.Y = dY;
         rc = launch_net<2, false>(q, a);
         if (rc) return rc;
-        HIPCHK(hipStreamSynchronize(q->stream));
-        return MST_OK;
+        return follow(stream, q->stream);
     }
     // rows in chunks of at most 1 << 20 through the work buffers
     const int64_t chunk = 1 << 20;
@@ -1367,6 +1381,7 @@ int mst_mlp_forward(mst_mlp *q, const float *X, int64_t n, float *Y) {
     if (hipMemcpy(dX, X, sizeof(float) * n * q->n_in, hipMemcpyHostToDevice) != hipSuccess)
         rc = mst::fail(MST_E_HIP, "copy failed");
     if (!rc) rc = mst::mlp_forward_device(q, dX, n, dY, q->stream);
+    if (!rc && hipStreamSynchronize(q->stream) != hipSuccess) rc = mst::fail(MST_E_HIP, "forward pass failed");
     if (!rc && hipMemcpy(Y, dY, sizeof(float) * n * q->n_out, hipMemcpyDeviceToHost) != hipSuccess)
         rc = mst::fail(MST_E_HIP, "copy failed");
     (void)hipFree(dX);

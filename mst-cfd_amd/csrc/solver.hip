@@ -564,6 +564,7 @@ void release(mst_ctx *x) {
             (void)hipEventDestroy(pr.second);
         }
     for (auto e : x->pool) (void)hipEventDestroy(e);
+    if (x->board) (void)hipHostFree(x->board);
     if (x->stream) (void)hipStreamDestroy(x->stream);
     delete x;
 }
@@ -573,12 +574,19 @@ int fetch_cells(mst_ctx *x, const double *dsrc, int width, double *out) {
     return MST_OK;
 }
 
+// scal and the bad flag on the board, after the stream's earlier work
+int report(mst_ctx *x, bool take_bad) {
+    hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, x->stream, (const double *)x->scal, x->bad, (int)take_bad, x->board,
+                       ++x->board_seq);
+    HIPCHK(hipGetLastError());
+    HIPCHK(board_wait(x->board, x->board_seq, x->stream));
+    return MST_OK;
+}
+
 int check_bad(mst_ctx *x) {
-    int h = 0;
-    HIPCHK(hipStreamSynchronize(x->stream));
-    HIPCHK(hipMemcpy(&h, x->bad, sizeof(int), hipMemcpyDeviceToHost));
-    if (h) {
-        HIPCHK(hipMemset(x->bad, 0, sizeof(int)));
+    int rc = report(x, true);
+    if (rc) return rc;
+    if (x->board->bad) {
         return mst::fail(MST_E_STATE, "non-physical state (rho<=0, p<=0 or NaN, or no positive time step) produced by the update");
     }
     return MST_OK;
@@ -944,6 +952,11 @@ int mst_ctx_create(const mst_mesh *m, const mst_config *cfg, mst_ctx **out) {
     for (int i = 0; i < 2; i++) TRY(dalloc(&x->pdt[i], x->nblk_c));
     TRY(dalloc(&x->fin_mid, 12 * (x->nblk_c / FIN_CHUNK + 2)));
     TRY(dalloc(&x->bad, 1));
+    if (hipHostMalloc((void **)&x->board, sizeof(Board), hipHostMallocCoherent) != hipSuccess) {
+        release(x);
+        return mst::fail(MST_E_HIP, "hipHostMalloc failed");
+    }
+    memset(x->board, 0, sizeof(Board));
     if (hipMemset(x->bad, 0, sizeof(int)) != hipSuccess || hipMemset(x->scal, 0, 16 * sizeof(double)) != hipSuccess ||
         hipMemset(x->rec, 0, sizeof(double) * x->slots * x->nc * x->nv) != hipSuccess) {
         release(x);
@@ -1001,8 +1014,8 @@ int mst_get_new_state(mst_ctx *ctx, double *Q, int64_t n_cells) {
 int mst_set_dt(mst_ctx *ctx, double dt) {
     CTX_GUARD(ctx);
     if (!(dt > 0)) return mst::fail(MST_E_ARG, "dt must be positive");
-    HIPCHK(hipMemcpyAsync(ctx->scal, &dt, sizeof(double), hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    hipLaunchKernelGGL(k_store, dim3(1), dim3(1), 0, ctx->stream, ctx->scal, dt);
+    HIPCHK(hipGetLastError());
     ctx->dt_valid = false;
     return MST_OK;
 }
@@ -1203,8 +1216,9 @@ int mst_compute_dt(mst_ctx *ctx, double cfl, double *dt) {
     if (!(cfl > 0) || !dt) return mst::fail(MST_E_ARG, "cfl must be positive");
     int rc = run_cfl(ctx, ctx->Q[ctx->iold], cfl);
     if (rc) return rc;
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    HIPCHK(hipMemcpy(dt, ctx->scal, sizeof(double), hipMemcpyDeviceToHost));
+    rc = report(ctx, false);
+    if (rc) return rc;
+    *dt = ctx->board->scal[0];
     ctx->dt_valid = cfl == ctx->cfg.cfl;
     if (!(*dt > 0)) return mst::fail(MST_E_STATE, "non-physical state: no positive CFL time step");
     return MST_OK;
@@ -1213,8 +1227,9 @@ int mst_compute_dt(mst_ctx *ctx, double cfl, double *dt) {
 int mst_residual_norms(mst_ctx *ctx, double *out) {
     CTX_GUARD(ctx);
     if (!out) return mst::fail(MST_E_ARG, "null argument");
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    HIPCHK(hipMemcpy(out, ctx->scal + 1, sizeof(double) * ctx->nv, hipMemcpyDeviceToHost));
+    int rc = report(ctx, false);
+    if (rc) return rc;
+    for (int k = 0; k < ctx->nv; k++) out[k] = ctx->board->scal[1 + k];
     return MST_OK;
 }
 
@@ -1226,20 +1241,16 @@ int mst_monitor_maxrel(mst_ctx *ctx, double *out) {
                           : launch(ctx, -1, k_maxrel<5>, ctx->nc, ctx->nc, (const double *)ctx->Q[ctx->inew],
                                    (const double *)ctx->Q[ctx->iold], ctx->part);
     if (rc) return rc;
-    FinArgs f;
-    memset(&f, 0, sizeof(f));
-    f.nblk = ctx->nblk_c;
-    f.count = 1.0;
-    for (int k = 0; k < ctx->nv; k++) {
-        f.src[k] = ctx->part + k * ctx->nblk_c;
-        f.kind[k] = 2;
-        f.dst[k] = ctx->scal + 6 + k;
-    }
-    f.n = ctx->nv;
-    rc = launch_finish(ctx, f);
-    if (rc) return rc;
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    HIPCHK(hipMemcpy(out, ctx->scal + 6, sizeof(double) * ctx->nv, hipMemcpyDeviceToHost));
+    const uint32_t seq = ++ctx->board_seq;
+    if (ctx->nv == 4)
+        hipLaunchKernelGGL(k_finish_max<4>, dim3(1), dim3(BLOCK), 0, ctx->stream, (const double *)ctx->part, ctx->nblk_c,
+                           ctx->board, seq);
+    else
+        hipLaunchKernelGGL(k_finish_max<5>, dim3(1), dim3(BLOCK), 0, ctx->stream, (const double *)ctx->part, ctx->nblk_c,
+                           ctx->board, seq);
+    HIPCHK(hipGetLastError());
+    HIPCHK(board_wait(ctx->board, seq, ctx->stream));
+    for (int k = 0; k < ctx->nv; k++) out[k] = ctx->board->mon[k];
     return MST_OK;
 }
 
@@ -1294,23 +1305,25 @@ int mst_ctx_warm_start(mst_ctx *ctx, mst_mlp *mlp, const double *cond, int n_con
     w.gamma = ctx->cfg.gamma;
     w.Q = ctx->Q[ctx->iold];
     w.bad = ctx->bad;
-    float *feat = nullptr, *out = nullptr;
-    HIPCHK(hipMalloc((void **)&feat, sizeof(float) * ctx->nc * n_in));
-    if (hipMalloc((void **)&out, sizeof(float) * ctx->nc * n_out) != hipSuccess) {
-        (void)hipFree(feat);
-        return mst::fail(MST_E_HIP, "hipMalloc failed");
-    }
+    // the two spare stage buffers hold the features and the outputs (nothing between calls)
+    int spare[2], ns = 0;
+    for (int i = 0; i < 4; i++)
+        if (i != ctx->iold && i != ctx->inew) spare[ns++] = i;
+    const bool fits = sizeof(float) * n_in <= sizeof(double) * ctx->nv;
+    float *feat = reinterpret_cast<float *>(ctx->Q[spare[0]]);
+    if (!fits) HIPCHK(hipMalloc((void **)&feat, sizeof(float) * ctx->nc * n_in));
     w.feat = feat;
-    w.Y = out;
+    w.Y = reinterpret_cast<float *>(ctx->Q[spare[1]]);
     int rc = ctx->dim == 2 ? launch(ctx, -1, k_warm_features<2>, ctx->nc, w) : launch(ctx, -1, k_warm_features<3>, ctx->nc, w);
-    if (!rc) rc = mst::mlp_forward_device(mlp, feat, ctx->nc, out, ctx->stream);
+    if (!rc) rc = mst::mlp_forward_device(mlp, feat, ctx->nc, reinterpret_cast<float *>(ctx->Q[spare[1]]), ctx->stream);
     if (!rc)
         rc = ctx->dim == 2 ? launch(ctx, -1, k_warm_decode<2>, ctx->nc, w) : launch(ctx, -1, k_warm_decode<3>, ctx->nc, w);
-    hipError_t e = hipStreamSynchronize(ctx->stream);
-    (void)hipFree(feat);
-    (void)hipFree(out);
+    if (!fits) {
+        const hipError_t e = hipStreamSynchronize(ctx->stream);
+        (void)hipFree(feat);
+        if (!rc && e != hipSuccess) return mst::fail(MST_E_HIP, hipGetErrorString(e));
+    }
     if (rc) return rc;
-    if (e != hipSuccess) return mst::fail(MST_E_HIP, hipGetErrorString(e));
     for (int i = 0; i < 4; i++) ctx->shadow_ok[i] = false;
     ctx->dt_valid = false;
     return check_bad(ctx);

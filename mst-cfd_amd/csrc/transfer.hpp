@@ -1,5 +1,5 @@
 // transfer.hpp -- cell records between a device array in the device's order and a caller's host array in
-// file order.
+// file order, and the few scalars of a step that the host waits for (Board, at the end).
 //
 // A kernel permutes straight into (or out of) pinned host memory, chunk by chunk, while the host copies the
 // chunk before to (or the chunk after from) the caller's pageable array.  What bounds it is the link: about
@@ -124,5 +124,43 @@ struct Transfer {
         return hipStreamSynchronize(st);
     }
 };
+
+// A context's results of a few words, in pinned host memory: a kernel behind the work stores them and then a sequence
+// number, which the host polls.  Waiting so takes 6 us from the launch, a stream synchronisation 11 and a copy into
+// pageable memory 11 more.
+struct Board {
+    double scal[16];
+    double mon[8];
+    int32_t bad;
+    uint32_t seq;
+};
+
+// scal and the bad flag to the board; take_bad: the flag is cleared as well
+static __global__ __launch_bounds__(64) void k_report(const double *__restrict__ scal, int *__restrict__ bad, int take_bad,
+                                                    Board *__restrict__ b, uint32_t seq) {
+    const int i = threadIdx.x;
+    if (i < 16) b->scal[i] = scal[i];
+    if (i == 16) {
+        const int v = bad[0];
+        b->bad = v;
+        if (take_bad && v) bad[0] = 0;
+    }
+    __threadfence_system();
+    __syncthreads();
+    if (i == 0) __hip_atomic_store(&b->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+static __global__ void k_store(double *__restrict__ p, double v) { p[0] = v; }
+
+// waits for board sequence number seq, the stream's newest: by polling for about 100 us, then on the stream
+inline hipError_t board_wait(const Board *b, uint32_t seq, hipStream_t st) {
+    for (int i = 0; i < 2048; i++) {
+        if (__atomic_load_n(&b->seq, __ATOMIC_ACQUIRE) == seq) return hipSuccess;
+        __builtin_ia32_pause();
+    }
+    const hipError_t e = hipStreamSynchronize(st);
+    if (e != hipSuccess) return e;
+    return __atomic_load_n(&b->seq, __ATOMIC_ACQUIRE) == seq ? hipSuccess : hipErrorUnknown;
+}
 
 }  // namespace mstk
