@@ -74,29 +74,34 @@ struct FluxArgs {
 // interior state and Y = its reconstructed face state for a boundary face, whose ghost combines the
 // two as the reference does.  Everything is read by face index, so the lanes of the two cells of a
 // face (cell strategy) load and then compute bit-identical states.
+// s0, s1: the face's entries of the side arrays (frec0, frec1 at order 2, else fc0, fc1).
 template <int DIM, bool SECOND, typename T>
-__device__ __forceinline__ void face_load(const FluxArgs<T> &a, int64_t f, int kind, double (&n64)[DIM],
-                                          T (&X)[DIM + 2], T (&Y)[DIM + 2]) {
+__device__ __forceinline__ void face_load(const FluxArgs<T> &a, int64_t f, int kind, int32_t s0, int32_t s1,
+                                          double (&n64)[DIM], T (&X)[DIM + 2], T (&Y)[DIM + 2]) {
     constexpr int NV = DIM + 2;
 #pragma unroll
     for (int d = 0; d < DIM; d++) n64[d] = a.fn[f * DIM + d];
     if (kind == mst::KIND_INTERIOR || kind == mst::KIND_PERIODIC) {
-        if constexpr (SECOND) {
-            ldq<NV>(a.rec + (int64_t)a.frec0[f] * NV, X);
-            ldq<NV>(a.rec + (int64_t)a.frec1[f] * NV, Y);
-        } else {
-            ldq<NV>(a.Q + (int64_t)a.fc0[f] * NV, X);
-            ldq<NV>(a.Q + (int64_t)a.fc1[f] * NV, Y);
-        }
+        const T *src = SECOND ? a.rec : a.Q;
+        ldq<NV>(src + (int64_t)s0 * NV, X);
+        ldq<NV>(src + (int64_t)s1 * NV, Y);
         return;
     }
-    ldq<NV>(a.Q + (int64_t)a.fc0[f] * NV, X);
+    ldq<NV>(a.Q + (int64_t)(SECOND ? a.fc0[f] : s0) * NV, X);
     if constexpr (SECOND) {
-        ldq<NV>(a.rec + (int64_t)a.frec0[f] * NV, Y);
+        ldq<NV>(a.rec + (int64_t)s0 * NV, Y);
     } else {
 #pragma unroll
         for (int k = 0; k < NV; k++) Y[k] = X[k];
     }
+}
+
+template <int DIM, bool SECOND, typename T>
+__device__ __forceinline__ void face_load(const FluxArgs<T> &a, int64_t f, int kind, double (&n64)[DIM],
+                                          T (&X)[DIM + 2], T (&Y)[DIM + 2]) {
+    const bool two = kind == mst::KIND_INTERIOR || kind == mst::KIND_PERIODIC;
+    const int32_t s0 = SECOND ? a.frec0[f] : a.fc0[f], s1 = two ? (SECOND ? a.frec1[f] : a.fc1[f]) : -1;
+    face_load<DIM, SECOND, T>(a, f, kind, s0, s1, n64, X, Y);
 }
 
 // Riemann left (A: c0 side) and right (B: c1 side or ghost) states from face_load's inputs; registers only
@@ -919,6 +924,13 @@ __device__ __forceinline__ void patch_sum(const double *g, int npf, const int (&
 // STAGE false: the residual only (R and, with a.l2, its norms), for the implicit steady driver.  NT lanes per patch of
 // BLOCK cells: twice as many on meshes of few patches, where the patch's faces then take one pass.  extra: what is
 // added to a face's flux (the viscous terms).
+// A lane has two or three faces, each a chain of loads (entry, the side's indices, the states) and a long solve: the
+// next face's indices are fetched while a face is solved, and the update's inputs before the barrier, where a wave waits
+// for the others anyway.  Microseconds per SSP-RK2 step before / with: first order 2D 12.9 / 11.7 (45,000 cells),
+// 57.8 / 56.8 (819,200); 3D Roe 23.2 / 22.3 (82,944), 80.7 / 78.9 (663,552); second order 3D AUSM 245.2 / 240.5 (the
+// patch kernel alone 62.4 / 55.4 in a profile).  Also fetching the next face's states (46 registers more), or the
+// update's inputs before the first face (22), is slower again from a few hundred patches on; so is a bound of 96
+// registers on 3D Roe (24 bytes of spill: 101 against 81).
 struct NoExtra {
     template <typename G>
     __device__ __forceinline__ void operator()(int64_t, int, G &) const {}
@@ -932,26 +944,42 @@ __global__ __launch_bounds__(NT) void k_patch(const FluxArgs<T> fa, const UpdArg
     const int64_t blk = block_id();
     const int32_t f0 = p.start[blk];
     const int npf = p.start[blk + 1] - f0;
-    for (int i = threadIdx.x; i < npf; i += NT) {
-        int64_t f;
+    const int64_t c = blk * BLOCK + threadIdx.x;
+    const bool valid = (NT == BLOCK || threadIdx.x < BLOCK) && c < a.nc;
+    struct Idx {
+        int32_t f;
         int info;
-        patch_face(p, fa.finfo, f0 + i, f, info);
-        double g[NV];
-        face_flux<DIM, SCHEME, SECOND, T>(fa, f, info & 15, info >> 4, g);
-        extra(f, info & 15, g);
+        int32_t s0, s1;
+    } nx;
+    auto fetch = [&](int i, Idx &x) {
+        int64_t f;
+        patch_face(p, fa.finfo, f0 + i, f, x.info);
+        x.f = (int32_t)f;
+        x.s0 = SECOND ? fa.frec0[f] : fa.fc0[f];
+        x.s1 = SECOND ? fa.frec1[f] : fa.fc1[f];
+    };
+    if ((int)threadIdx.x < npf) fetch(threadIdx.x, nx);
+    for (int i = threadIdx.x; i < npf; i += NT) {
+        const Idx x = nx;
+        double g[NV], n64[DIM];
+        T X[NV], Y[NV];
+        face_load<DIM, SECOND, T>(fa, x.f, x.info & 15, x.s0, x.s1, n64, X, Y);
+        if (i + NT < npf) fetch(i + NT, nx);
+        face_solve<DIM, SCHEME, T>(fa.P, SCHEME == MST_SCHEME_ROE, x.info & 15, x.info >> 4, n64, X, Y, g);
+        extra(x.f, x.info & 15, g);
 #pragma unroll
         for (int k = 0; k < NV; k++) gsh[k * npf + i] = g[k];
     }
-    const double dt = STAGE ? stage_dt(a) : 0.0;
-    __syncthreads();
-    const int64_t c = blk * BLOCK + threadIdx.x;
-    const bool valid = (NT == BLOCK || threadIdx.x < BLOCK) && c < a.nc;
     int cl[MAXF];
 #pragma unroll
     for (int s = 0; s < MAXF; s++) cl[s] = valid ? p.loc[(int64_t)s * a.nc + c] : -1;  // padded to MAXF rows
+    StageIn<NV> in;
+    if (STAGE && valid) stage_load<NV, F32>(a, c, in);
+    const double dt = STAGE ? stage_dt(a) : 0.0;
+    __syncthreads();
     double r[NV];
     patch_sum<NV, MAXF, F32>(gsh, npf, cl, r);
-    stage_tail<NV, STAGE, F32, NT>(a, c, valid, dt, r, blk, a.l2, a.dtred);
+    stage_tail<NV, STAGE, F32, NT>(a, c, valid, dt, r, blk, a.l2, a.dtred, STAGE ? &in : nullptr);
 }
 
 // Order 2 in one kernel: the patch also computes the limited gradients of its own cells and of its
@@ -1167,11 +1195,13 @@ __global__ __launch_bounds__(NT) void k_patch_rec(const FluxArgs<float> fa, cons
 #pragma unroll
         for (int k = 0; k < NV; k++) L.g[k * npf + i] = g[k];
     }
+    StageIn<NV> in;
+    if (valid) stage_load<NV, true>(a, c, in);
     const double dt = stage_dt(a);
     __syncthreads();
     double r[NV];
     patch_sum<NV, MAXF, true>(L.g, npf, cl, r);
-    stage_tail<NV, true, true, NT>(a, c, valid, dt, r, blk, a.l2, a.dtred);
+    stage_tail<NV, true, true, NT>(a, c, valid, dt, r, blk, a.l2, a.dtred, &in);
 }
 
 // Resident waves per SIMD requested for the fused kernel, where the bound costs no more than a register

@@ -19,17 +19,21 @@ int run_patch_t(mst_ctx *x, int mode, int is, int in, const Stage &sg, int iout)
     const bool roe = x->cfg.scheme == MST_SCHEME_ROE;
     if (x->viscous) {
         const ViscFace<DIM> vf{visc_args(x, is)};
-#define MST_PATCH_V(MF, SECOND)                                                                                             \
-    return roe ? launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_ROE, SECOND, T, MF, true, BLOCK, ViscFace<DIM>>, x->nc, \
-                           BLOCK, shm, fa, a, pa, vf)                                                                       \
-               : launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_AUSM, SECOND, T, MF, true, BLOCK, ViscFace<DIM>>, x->nc, \
-                           BLOCK, shm, fa, a, pa, vf);
+#define MST_PATCH_V_N(MF, SECOND, NT)                                                                                       \
+    return roe ? launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_ROE, SECOND, T, MF, true, NT, ViscFace<DIM>>, x->nc, NT, \
+                           shm, fa, a, pa, vf)                                                                              \
+               : launch_nt(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_AUSM, SECOND, T, MF, true, NT, ViscFace<DIM>>, x->nc,    \
+                           NT, shm, fa, a, pa, vf);
+#define MST_PATCH_V(MF, SECOND)                                 \
+    if (x->wide_patch) { MST_PATCH_V_N(MF, SECOND, 2 * BLOCK) } \
+    MST_PATCH_V_N(MF, SECOND, BLOCK)
         if (x->slots == 3) {
             if (second) { MST_PATCH_V(3, true) }
             MST_PATCH_V(3, false)
         }
         if (second) { MST_PATCH_V(4, true) }
         MST_PATCH_V(4, false)
+#undef MST_PATCH_V_N
 #undef MST_PATCH_V
     }
     if constexpr (std::is_same<T, float>::value) {
