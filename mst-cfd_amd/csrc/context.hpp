@@ -46,7 +46,7 @@ struct mst_ctx {
     int iold = 0, inew = 1;
     double *G = nullptr, *rec = nullptr, *graw = nullptr, *phi = nullptr, *R = nullptr;
     int32_t *frec0 = nullptr, *frec1 = nullptr;  // incidence records of each face's c0 / c1 side
-    // patch strategy: per block of BLOCK cells its flux-carrying faces, per cell slot the local index
+    // patch strategy: per patch of patch_cells cells its flux-carrying faces, per cell slot the local index
     int32_t *pstart = nullptr, *pface = nullptr;
     int16_t *ploc = nullptr;
     uint32_t *pfi = nullptr;  // pface with the faces' kinds and L/R masks packed in (null: 2^26 faces or more)
@@ -84,6 +84,16 @@ struct mst_ctx {
     // 66 / 76 (324); first-order patch 2D 14.0 / 13.3 (176), 16.6 / 16.6 (313), 21.9 / 23.5 (704); patch 3D
     // 36 / 32 (41), 57.0 / 54.4 (324), 80.3 / 80.9 (633).
     bool wide_patch = false, wide_fused = false;
+    // Patches of SUB_PATCH cells where those of BLOCK cells would leave most of the chip idle: a stage's time is then
+    // one patch's, and a patch of 64 cells is one wave of each phase's work on its compute unit instead of four (two in
+    // a row on each SIMD).  One small patch per CU in 3D, two in 2D: beyond that their larger halo costs more.
+    // Microseconds per step, wide patches / small ones, by blocks of BLOCK cells: fused 2D 20.3 / 16.4 (32), 20.5 /
+    // 18.8 (95), 20.6 / 20.2 (133); first order 2D 11.4 / 9.9 (32), 11.8 / 11.7 (113), 12.0 / 13.2 (133); viscous 2D
+    // 24.6 / 22.8 (32), 26.5 / 25.9 (113), 26.9 / 28.2 (133); patch 3D 31.2 / 29.2 (32), 31.6 / 29.8 (52), 32.4 /
+    // 32.7 (80); first order 3D 17.0 / 15.8 (52), 17.1 / 17.7 (65); the mixed form in 3D 28.7 / 29.3 (24), so not there.
+    int patch_cells = BLOCK;  // BLOCK or SUB_PATCH
+    int64_t n_patch = 0;
+    int64_t dt_cnt[2] = {0, 0}, l2_cnt = 0;  // partials in pdt[i] and part, as their last writer left them
     int *bad = nullptr;
     Board *board = nullptr;  // pinned: the words the host waits for
     uint32_t board_seq = 0;
@@ -147,6 +157,12 @@ int launch_nt(mst_ctx *x, int kclass, K kernel, int64_t n, int nt, size_t shm, A
     return MST_OK;
 }
 
+// a kernel over the patches, nt lanes each
+template <typename K, typename... Args>
+int launch_patch(mst_ctx *x, int kclass, K kernel, int nt, size_t shm, Args... args) {
+    return launch_nt(x, kclass, kernel, x->n_patch * BLOCK, nt, shm, args...);
+}
+
 template <typename K, typename... Args>
 int launch(mst_ctx *x, int kclass, K kernel, int64_t nthreads, Args... args) {
     return launch_nt(x, kclass, kernel, nthreads, BLOCK, 0, args...);
@@ -200,6 +216,12 @@ FluxArgs<T> flux_args(const mst_ctx *x, int isrc) {
     return a;
 }
 
+// the launch that follows writes n partials of what mode reduces
+inline void partials(mst_ctx *x, int mode, int64_t n) {
+    if (mode & UPD_DT) x->dt_cnt[x->dt_to] = n;
+    if (mode & UPD_L2) x->l2_cnt = n;
+}
+
 inline UpdArgs upd_args(const mst_ctx *x, int mode, int is, int in, const Stage &sg, int iout) {
     UpdArgs a;
     a.nc = x->nc;
@@ -211,7 +233,7 @@ inline UpdArgs upd_args(const mst_ctx *x, int mode, int is, int in, const Stage 
     a.sh = x->cshalf;
     a.dt = x->scal;
     a.dt_part = x->dt_from >= 0 ? x->pdt[x->dt_from] : nullptr;
-    a.dt_n = x->dt_from >= 0 ? (int)x->nblk_c : 0;
+    a.dt_n = x->dt_from >= 0 ? (int)x->dt_cnt[x->dt_from] : 0;
     set_stage(a, sg);
     a.maxf = x->maxf;
     a.l2 = (mode & UPD_L2) != 0;

@@ -9,6 +9,7 @@
 namespace mstk {
 
 constexpr int BLOCK = 256;
+constexpr int SUB_PATCH = 64;  // cells of a patch on small meshes
 
 // physical and reference constants in the arithmetic type of the kernel
 template <typename T>

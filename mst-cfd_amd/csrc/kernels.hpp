@@ -922,7 +922,7 @@ __device__ __forceinline__ void patch_sum(const double *g, int npf, const int (&
 }
 
 // STAGE false: the residual only (R and, with a.l2, its norms), for the implicit steady driver.  NT lanes per patch of
-// BLOCK cells: twice as many on meshes of few patches, where the patch's faces then take one pass.  extra: what is
+// PC cells: twice as many on meshes of few patches, where the patch's faces then take one pass.  extra: what is
 // added to a face's flux (the viscous terms).
 // A lane has two or three faces, each a chain of loads (entry, the side's indices, the states) and a long solve: the
 // next face's indices are fetched while a face is solved, and the update's inputs before the barrier, where a wave waits
@@ -935,7 +935,8 @@ struct NoExtra {
     template <typename G>
     __device__ __forceinline__ void operator()(int64_t, int, G &) const {}
 };
-template <int DIM, int SCHEME, bool SECOND, typename T, int MAXF, bool STAGE = true, int NT = BLOCK, typename Extra = NoExtra>
+template <int DIM, int SCHEME, bool SECOND, typename T, int MAXF, bool STAGE = true, int PC = BLOCK, int NT = PC,
+          typename Extra = NoExtra>
 __global__ __launch_bounds__(NT) void k_patch(const FluxArgs<T> fa, const UpdArgs a, const PatchArgs p,
                                               const Extra extra = Extra()) {
     constexpr int NV = DIM + 2;
@@ -944,8 +945,8 @@ __global__ __launch_bounds__(NT) void k_patch(const FluxArgs<T> fa, const UpdArg
     const int64_t blk = block_id();
     const int32_t f0 = p.start[blk];
     const int npf = p.start[blk + 1] - f0;
-    const int64_t c = blk * BLOCK + threadIdx.x;
-    const bool valid = (NT == BLOCK || threadIdx.x < BLOCK) && c < a.nc;
+    const int64_t c = blk * PC + threadIdx.x;
+    const bool valid = (NT == PC || threadIdx.x < PC) && c < a.nc;
     struct Idx {
         int32_t f;
         int info;
@@ -1130,7 +1131,7 @@ inline size_t fused_lds_bytes(int dim, int nv, int max_pf, bool f32, bool staged
 // each record once per patch; the inputs of every face's solve are the records k_flux would read, so
 // the results are bit-identical.  LDS: the fused kernel's FP32 layout, 8 * NV bytes per face (the
 // size of the FP64 fluxes that overwrite them).
-template <int DIM, int SCHEME, int MAXF, int NT = BLOCK>
+template <int DIM, int SCHEME, int MAXF, int PC = BLOCK, int NT = PC>
 __global__ __launch_bounds__(NT) void k_patch_rec(const FluxArgs<float> fa, const UpdArgs a, const PatchArgs p,
                                                      const HaloArgs h) {
     constexpr int NV = DIM + 2;
@@ -1139,8 +1140,8 @@ __global__ __launch_bounds__(NT) void k_patch_rec(const FluxArgs<float> fa, cons
     const int32_t f0 = p.start[blk];
     const int npf = p.start[blk + 1] - f0;
     FusedLds<float> L(gsh, npf, NV);
-    const int64_t c = blk * BLOCK + threadIdx.x;
-    const bool valid = (NT == BLOCK || threadIdx.x < BLOCK) && c < a.nc;
+    const int64_t c = blk * PC + threadIdx.x;
+    const bool valid = (NT == PC || threadIdx.x < PC) && c < a.nc;
     int cl[MAXF];
 #pragma unroll
     for (int s = 0; s < MAXF; s++) cl[s] = valid ? p.loc[(int64_t)s * a.nc + c] : -1;
@@ -1156,8 +1157,8 @@ __global__ __launch_bounds__(NT) void k_patch_rec(const FluxArgs<float> fa, cons
         for (int k = 0; k < NV; k++) L.r(l & 1, k, l >> 1, NV) = q[k];
     }
     // (lanes past the patch's cells take the halo beside them)
-    for (int j = NT > BLOCK ? (int)threadIdx.x - BLOCK : threadIdx.x; j < nh; j += NT > BLOCK ? NT - BLOCK : BLOCK) {
-        if (NT > BLOCK && j < 0) break;
+    for (int j = NT > PC ? (int)threadIdx.x - PC : threadIdx.x; j < nh; j += NT > PC ? NT - PC : NT) {
+        if (NT > PC && j < 0) break;
         const int64_t hc = h.cell[h0 + j];
 #pragma unroll
         for (int s = 0; s < MAXF; s++) {
@@ -1222,9 +1223,9 @@ constexpr int fused_waves() {
 // entries ((local face << 1) | side, -1: none) for the caller's sums.  roe picks the scheme when
 // SCHEME is SCHEME_RUNTIME.  pre() runs between the gradient and the flux phases, when the gradient's
 // registers are free: the caller fetches its update's inputs there, so their latency overlaps the
-// face solves.  NT = 2 BLOCK: the lanes past the patch's cells take the halo's gradients at the same time, and
+// face solves.  NT = 2 PC: the lanes past the patch's cells take the halo's gradients at the same time, and
 // the patch's faces take one pass.
-template <int DIM, int SCHEME, int LIM, typename T, int MAXF, bool NRM_LDS = false, int NT = BLOCK, typename Pre>
+template <int DIM, int SCHEME, int LIM, typename T, int MAXF, bool NRM_LDS = false, int PC = BLOCK, int NT = PC, typename Pre>
 __device__ __forceinline__ void fused_patch(const GradArgs<T> &ga, const FluxArgs<T> &fa, bool roe, const PatchArgs &p,
                                             const HaloArgs &h, int64_t patch, int64_t cb, int64_t ce, int64_t nc,
                                             int32_t f0, FusedLds<T> &L, int (&cl)[MAXF], Pre pre) {
@@ -1233,7 +1234,7 @@ __device__ __forceinline__ void fused_patch(const GradArgs<T> &ga, const FluxArg
     // Inputs of the later phases that do not depend on the gradients are fetched first, so their
     // latency overlaps the gradient phase: each lane's first PF patch faces (face, kind, normal), its
     // cell's slot entries and its first halo cell.
-    constexpr int PF = NT > BLOCK ? 1 : MST_FUSED_PF;
+    constexpr int PF = NT > PC ? 1 : MST_FUSED_PF;
     int64_t pf_f[PF];
     int pf_info[PF];
     double pf_n[PF][DIM];
@@ -1249,15 +1250,15 @@ __device__ __forceinline__ void fused_patch(const GradArgs<T> &ga, const FluxArg
         }
     }
     const int64_t c = cb + threadIdx.x;
-    const bool mine = (NT == BLOCK || threadIdx.x < BLOCK) && c < ce;
+    const bool mine = (NT == PC || threadIdx.x < PC) && c < ce;
 #pragma unroll
     for (int s = 0; s < MAXF; s++) cl[s] = mine ? p.loc[(int64_t)s * nc + c] : -1;
     // limited gradients of the patch cells, then of the halo cells; face states into LDS
     const int32_t h0 = h.start[patch];
-    const int next = BLOCK + (h.start[patch + 1] - h0);  // the patch's cells, then its halo
+    const int next = PC + (h.start[patch + 1] - h0);  // the patch's cells, then its halo
     // the lane's first halo cell (a wide block: of the lanes past the patch's cells)
-    const int j0 = NT > BLOCK ? (int)threadIdx.x - BLOCK : (int)threadIdx.x;
-    const int32_t hc = (NT == BLOCK || j0 >= 0) && BLOCK + j0 < next ? h.cell[h0 + j0] : 0;
+    const int j0 = NT > PC ? (int)threadIdx.x - PC : (int)threadIdx.x;
+    const int32_t hc = (NT == PC || j0 >= 0) && PC + j0 < next ? h.cell[h0 + j0] : 0;
     const IncView<T> own = cell_view(ga);
     const IncView<T> hv{h.code, static_cast<const T *>(h.w), static_cast<const T *>(h.n),
                         static_cast<const T *>(h.dx), static_cast<const GradVol<T> *>(h.vol), h.nh};
@@ -1313,14 +1314,14 @@ __device__ __forceinline__ void fused_patch(const GradArgs<T> &ga, const FluxArg
             }
         }
     }
-    for (int i0 = NRM_LDS && NT == BLOCK ? BLOCK : 0; i0 < next; i0 += NT) {
+    for (int i0 = NRM_LDS && NT == PC ? PC : 0; i0 < next; i0 += NT) {
         const int i = i0 + (int)threadIdx.x;
         if (i >= next) break;
-        if (NRM_LDS && NT > BLOCK && i < BLOCK) continue;  // done above
+        if (NRM_LDS && NT > PC && i < PC) continue;  // done above
         int64_t cc, g;
         const int16_t *lp;
         int64_t stride;
-        const bool halo = NT == BLOCK ? i0 > 0 : i >= BLOCK;
+        const bool halo = NT == PC ? i0 > 0 : i >= PC;
         if (!halo) {
             cc = cb + i;
             if (cc >= ce) continue;
@@ -1328,8 +1329,8 @@ __device__ __forceinline__ void fused_patch(const GradArgs<T> &ga, const FluxArg
             lp = p.loc + cc;
             stride = nc;
         } else {
-            g = h0 + i - BLOCK;
-            cc = i < 2 * BLOCK ? hc : h.cell[g];
+            g = h0 + i - PC;
+            cc = i < 2 * PC ? hc : h.cell[g];
             lp = h.loc + g * MAXF;
             stride = 1;
         }
@@ -1393,8 +1394,8 @@ __device__ __forceinline__ void fused_patch(const GradArgs<T> &ga, const FluxArg
     __syncthreads();
 }
 
-template <int DIM, int SCHEME, int LIM, typename T, int MAXF, int NT = BLOCK>
-__global__ __launch_bounds__(NT, (NT > BLOCK ? 2 : fused_waves<DIM, SCHEME, LIM, T, MAXF>())) void k_fused(
+template <int DIM, int SCHEME, int LIM, typename T, int MAXF, int PC = BLOCK, int NT = PC>
+__global__ __launch_bounds__(NT, (NT > PC ? 2 : fused_waves<DIM, SCHEME, LIM, T, MAXF>())) void k_fused(
     const GradArgs<T> ga, const FluxArgs<T> fa, const UpdArgs a, const PatchArgs p, const HaloArgs h) {
     constexpr int NV = DIM + 2;
     constexpr bool F32 = std::is_same<T, float>::value;
@@ -1402,13 +1403,13 @@ __global__ __launch_bounds__(NT, (NT > BLOCK ? 2 : fused_waves<DIM, SCHEME, LIM,
     const int64_t blk = block_id();
     const int32_t f0 = p.start[blk];
     FusedLds<T> L(sh, p.start[blk + 1] - f0, NV);
-    const int64_t cb = blk * BLOCK, ce = cb + BLOCK < a.nc ? cb + BLOCK : a.nc;
+    const int64_t cb = blk * PC, ce = cb + PC < a.nc ? cb + PC : a.nc;
     int cl[MAXF];
     const int64_t c = cb + threadIdx.x;
-    const bool valid = (NT == BLOCK || threadIdx.x < BLOCK) && c < a.nc;
+    const bool valid = (NT == PC || threadIdx.x < PC) && c < a.nc;
     StageIn<NV> in;
     double dt = 0;
-    fused_patch<DIM, SCHEME, LIM, T, MAXF, fused_lds_normals<DIM>(), NT>(ga, fa, SCHEME == MST_SCHEME_ROE, p, h, blk, cb,
+    fused_patch<DIM, SCHEME, LIM, T, MAXF, fused_lds_normals<DIM>(), PC, NT>(ga, fa, SCHEME == MST_SCHEME_ROE, p, h, blk, cb,
                                                                           ce, a.nc, f0, L, cl, [&]() {
         dt = stage_dt(a);
         if (valid) stage_load<NV, F32>(a, c, in);
@@ -1469,6 +1470,20 @@ __global__ __launch_bounds__(BLOCK) void k_maxrel(int64_t nc, const double *__re
         __syncthreads();
     }
     if (threadIdx.x < NV) part[threadIdx.x * (int64_t)gridDim.x + blk] = s[threadIdx.x][0];
+}
+
+// part[k][b] = the sum of the partials of block b's SUB_PATCH patches in order (n patches), which is the partial of
+// a block of BLOCK cells bit for bit: block_partial adds its waves' sums in this order
+template <int U>
+__global__ __launch_bounds__(BLOCK) void k_join_partials(int64_t n, int64_t nb, int nv, const double *__restrict__ sub,
+                                                         double *__restrict__ part) {
+    const int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
+    if (i >= nb * nv) return;
+    const int64_t k = i / nb, b = i % nb;
+    constexpr int R = BLOCK / SUB_PATCH;
+    double v = sub[k * n + b * R];
+    for (int r = 1; r < R && b * R + r < n; r++) v += sub[k * n + b * R + r];
+    part[i] = v;
 }
 
 // Finish of the per-block partials.  Slot k is a sum (kind 0), a min (kind 1) or a max (kind 2).

@@ -143,6 +143,7 @@ int run_face_flux(mst_ctx *x, int isrc) {
 template <int NV, bool GT>
 int run_update_t(mst_ctx *x, int mode, int is, int in, const Stage &sg, int iout) {
     const UpdArgs a = upd_args(x, mode, is, in, sg, iout);
+    partials(x, mode, x->nblk_c);
 #define MST_UPD(MF)                                                                                             \
     switch (mode & ~UPD_CHECK) {                                                                                             \
         case UPD_RESIDUAL: return launch(x, MST_K_UPDATE, k_update<NV, MF, UPD_RESIDUAL, GT>, x->nc, a);        \
@@ -176,6 +177,7 @@ template <int DIM, typename T>
 int run_cell_t(mst_ctx *x, int mode, int is, int in, const Stage &sg, int iout) {
     const FluxArgs<T> fa = flux_args<T>(x, is);
     const UpdArgs a = upd_args(x, mode, is, in, sg, iout);
+    partials(x, mode, x->nblk_c);
     const bool second = x->cfg.order >= 2;
     const bool roe = x->cfg.scheme == MST_SCHEME_ROE;
     // slot count of the padded slot-major table: 3 (triangles), 4 (quadrilaterals, tetrahedra), 8
@@ -279,21 +281,38 @@ int launch_finish(mst_ctx *x, FinArgs f) {
     return MST_OK;
 }
 
-// one finish: L2 norms (nl2 fields) and/or the minimum time step, from the per-block partials
+// one finish: L2 norms (nl2 fields) and/or the minimum time step, from the per-block partials.  The norms are always
+// sums over the partials of blocks of BLOCK cells, whichever patches the kernel had.
 int run_finish(mst_ctx *x, int nl2, int want_dt) {
     FinArgs f;
     memset(&f, 0, sizeof(f));
     const int64_t nb = x->nblk_c;
     f.nblk = nb;
     f.count = (double)x->nc;
+    const double *part = x->part;
+    if (nl2 && x->l2_cnt != nb) {
+        double *joined = x->part + x->n_patch * x->nv;
+        hipLaunchKernelGGL(k_join_partials<0>, dim3((uint32_t)((nb * nl2 + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, x->stream,
+                           x->l2_cnt, nb, nl2, part, joined);
+        HIPCHK(hipGetLastError());
+        part = joined;
+    }
     for (int k = 0; k < nl2; k++) {
-        f.src[f.n] = x->part + k * nb;
+        f.src[f.n] = part + k * nb;
         f.kind[f.n] = 0;
         f.dst[f.n] = x->scal + 1 + k;
         f.post[f.n] = 1;
         f.n++;
     }
     if (want_dt) {
+        const int64_t nd = x->dt_cnt[x->dt_to];
+        if (nl2 && nd != nb) {  // the partials of other blocks: a finish of its own
+            int rc = launch_finish(x, f);
+            if (rc) return rc;
+            memset(&f, 0, sizeof(f));
+            f.count = (double)x->nc;
+        }
+        f.nblk = nd;
         f.src[f.n] = x->pdt[x->dt_to];
         f.kind[f.n] = 1;
         f.dst[f.n] = x->scal;
@@ -305,6 +324,7 @@ int run_finish(mst_ctx *x, int nl2, int want_dt) {
 
 int run_cfl(mst_ctx *x, const double *Qsrc, double cfl) {
     double *pdt = x->pdt[x->dt_to];
+    partials(x, UPD_DT, x->nblk_c);
     int rc = x->dim == 2 ? launch(x, MST_K_DT, k_cfl<2>, x->nc, x->nc, Qsrc, (const double *)x->cvol,
                                   (const double *)x->cshalf, x->cfg.gamma, cfl, pdt)
                          : launch(x, MST_K_DT, k_cfl<3>, x->nc, x->nc, Qsrc, (const double *)x->cvol,
@@ -368,7 +388,7 @@ int build_incidence(mst_ctx *x) {
     return rc;
 }
 
-// Patch tables: for each block of BLOCK consecutive cells, the faces that carry a flux into one of its
+// Patch tables: for each patch of patch_cells consecutive cells, the faces that carry a flux into one of its
 // cells (ascending; a face joining two of its cells once), and for each cell slot (local index << 1) |
 // is_c1, or -1 for an empty slot or a zero-flux face; and each patch's halo for the fused kernel.
 // The kernels keep a patch's face states and fluxes in LDS, so the strategies need at most 4 slots and
@@ -377,13 +397,12 @@ int build_patches(mst_ctx *x) {
     const mst::Prepared &P = x->prep.P;
     x->patch_ok = x->fused_ok = false;
     if (x->slots > 4) return MST_OK;
-    const int64_t nc = x->nc, nb = (nc + BLOCK - 1) / BLOCK;
+    const int64_t nc = x->nc, pc = x->patch_cells, nb = x->n_patch;
     std::vector<int32_t> start(nb + 1, 0), face, list, hstart(nb + 1, 0), hcell, halo;
     std::vector<int16_t> loc((size_t)x->slots * nc, -1), hloc;
     face.reserve((size_t)(nc * 2));
-    size_t max_pf = 0;
-    for (int64_t b = 0; b < nb; b++) {
-        const int64_t ca = b * BLOCK, cz = std::min(nc, ca + BLOCK);
+    size_t max_pf = 0, max_bf = 0;
+    auto faces_of = [&](int64_t ca, int64_t cz) {  // list = the flux-carrying faces of cells [ca, cz)
         list.clear();
         for (int s = 0; s < P.maxf; s++)
             for (int64_t c = ca; c < cz; c++) {
@@ -392,6 +411,16 @@ int build_patches(mst_ctx *x) {
             }
         std::sort(list.begin(), list.end());
         list.erase(std::unique(list.begin(), list.end()), list.end());
+    };
+    for (int64_t ca = 0; ca < nc; ca += BLOCK) {  // what a mesh may run does not depend on the size of its patches
+        faces_of(ca, std::min<int64_t>(nc, ca + BLOCK));
+        max_bf = std::max(max_bf, list.size());
+    }
+    // the fused kernel keeps 16 * NV bytes per patch face in LDS (the patch kernel half of that)
+    if (max_bf * x->nv * 16 > 65536) return MST_OK;
+    for (int64_t b = 0; b < nb; b++) {
+        const int64_t ca = b * pc, cz = std::min(nc, ca + pc);
+        faces_of(ca, cz);
         max_pf = std::max(max_pf, list.size());
         for (int s = 0; s < P.maxf; s++)
             for (int64_t c = ca; c < cz; c++) {
@@ -428,8 +457,6 @@ int build_patches(mst_ctx *x) {
     }
     start[nb] = (int32_t)face.size();
     hstart[nb] = (int32_t)hcell.size();
-    // the fused kernel keeps 16 * NV bytes per patch face in LDS (the patch kernel half of that)
-    if (max_pf * x->nv * 16 > 65536) return MST_OK;
     int rc = dupload(&x->pstart, start);
     if (!rc) rc = dupload(&x->pface, face);
     if (!rc && x->nf < ((int64_t)1 << FI_SHIFT)) rc = dalloc(&x->pfi, face.size());  // packed by upload_config
@@ -442,7 +469,7 @@ int build_patches(mst_ctx *x) {
     x->max_pf = (int)max_pf;
     x->n_psolve = (int64_t)face.size();
     x->patch_ok = true;
-    x->fused_ok = fused_lds_bytes(x->dim, x->nv, x->max_pf, false, x->dim == 2) <= 65536;
+    x->fused_ok = fused_lds_bytes(x->dim, x->nv, (int)max_bf, false, x->dim == 2) <= 65536;
     return MST_OK;
 }
 
@@ -909,6 +936,9 @@ int mst_ctx_create(const mst_mesh *m, const mst_config *cfg, mst_ctx **out) {
     x->nblk_f = (x->nf + BLOCK - 1) / BLOCK;
     x->wide_patch = x->nblk_c <= (x->dim == 3 ? 512 : 256);
     x->wide_fused = x->nblk_c <= (x->dim == 2 ? 512 : 256);
+    x->patch_cells = x->nblk_c <= (x->dim == 2 ? 128 : 64) && (x->dim == 2 || cfg->precision != MST_PREC_MIXED) ? SUB_PATCH
+                                                                                                           : BLOCK;
+    x->n_patch = (x->nc + x->patch_cells - 1) / x->patch_cells;
 #define TRY(e)            \
     do {                  \
         int _r = (e);     \
@@ -955,8 +985,8 @@ int mst_ctx_create(const mst_mesh *m, const mst_config *cfg, mst_ctx **out) {
     TRY(dalloc(&x->G, x->nf * x->nv));
     TRY(dalloc(&x->rec, (int64_t)x->slots * x->nc * x->nv));
     TRY(dalloc(&x->scal, 16));
-    TRY(dalloc(&x->part, std::max(x->nblk_c, x->nblk_f) * x->nv + 16));
-    for (int i = 0; i < 2; i++) TRY(dalloc(&x->pdt[i], x->nblk_c));
+    TRY(dalloc(&x->part, std::max(x->n_patch + x->nblk_c, x->nblk_f) * x->nv + 16));
+    for (int i = 0; i < 2; i++) TRY(dalloc(&x->pdt[i], std::max(x->n_patch, x->nblk_c)));
     TRY(dalloc(&x->fin_mid, 12 * (x->nblk_c / FIN_CHUNK + 2)));
     TRY(dalloc(&x->bad, 1));
     if (hipHostMalloc((void **)&x->board, sizeof(Board), hipHostMallocCoherent) != hipSuccess) {
@@ -1074,7 +1104,7 @@ int mst_update_new_to_old(mst_ctx *ctx) {
 }
 
 // Blocks up to which a step's stages reduce the block minima of its time step (stage_dt) instead of a launch between
-// the steps.  Microseconds per SSP-RK2 step, launch / in the stages: 24.7 / 23.6 at 32 blocks, 18.4 / 17.0 at 512 (first
+// the steps (patches of SUB_PATCH cells count).  Microseconds per SSP-RK2 step, launch / in the stages: 24.7 / 23.6 at 32 blocks, 18.4 / 17.0 at 512 (first
 // order), 26.5 / 27.2 at 1013.
 constexpr int64_t STEP_DT_MAX = 512;
 
@@ -1123,7 +1153,7 @@ int mst_step(mst_ctx *ctx, int nsteps) {
         }
         // the next step's time step: on meshes of few blocks its stages reduce the minima themselves
         ctx->dt_from = -1;
-        if (!rc && cfl && !l2 && ctx->nblk_c <= STEP_DT_MAX)
+        if (!rc && cfl && !l2 && ctx->dt_cnt[ctx->dt_to] <= STEP_DT_MAX)
             ctx->dt_from = ctx->dt_to;
         else if (!rc && (l2 || cfl))
             rc = run_finish(ctx, l2 ? ctx->nv : 0, cfl ? 1 : 0);

@@ -25,6 +25,7 @@ int run_fused_t(mst_ctx *x, int mode, int is, int in, const Stage &sg, int iout)
     const GradArgs<T> ga = grad_args<T>(x, is, false);
     const FluxArgs<T> fa = flux_args<T>(x, is);
     const UpdArgs a = upd_args(x, mode, is, in, sg, iout);
+    partials(x, mode, x->n_patch);
     PatchArgs pa;
     pa.start = x->pstart;
     pa.face = x->pface;
@@ -43,9 +44,12 @@ int run_fused_t(mst_ctx *x, int mode, int is, int in, const Stage &sg, int iout)
     const bool roe = x->cfg.scheme == MST_SCHEME_ROE;
     const int lim = x->cfg.limiter;
 #define MST_FUSED_L(SC, LM, MF)                                                                                         \
-    return x->wide_fused                                                                                                      \
-               ? launch_nt(x, MST_K_FUSED, k_fused<DIM, SC, LM, T, MF, 2 * BLOCK>, x->nc, 2 * BLOCK, shm, ga, fa, a, pa, ha) \
-               : launch_nt(x, MST_K_FUSED, k_fused<DIM, SC, LM, T, MF>, x->nc, BLOCK, shm, ga, fa, a, pa, ha);
+    if (x->patch_cells == SUB_PATCH)                                                                                    \
+        return launch_patch(x, MST_K_FUSED, k_fused<DIM, SC, LM, T, MF, SUB_PATCH, 2 * SUB_PATCH>, 2 * SUB_PATCH, shm,  \
+                            ga, fa, a, pa, ha);                                                                         \
+    return x->wide_fused ? launch_patch(x, MST_K_FUSED, k_fused<DIM, SC, LM, T, MF, BLOCK, 2 * BLOCK>, 2 * BLOCK, shm,  \
+                                        ga, fa, a, pa, ha)                                                              \
+                         : launch_patch(x, MST_K_FUSED, k_fused<DIM, SC, LM, T, MF>, BLOCK, shm, ga, fa, a, pa, ha);
 #define MST_FUSED_S(SC, MF)                                                                   \
     if (lim == MST_LIM_NONE) { MST_FUSED_L(SC, MST_LIM_NONE, MF) }                            \
     if (lim == MST_LIM_MINMOD) { MST_FUSED_L(SC, MST_LIM_MINMOD, MF) }                        \
