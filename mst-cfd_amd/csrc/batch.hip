@@ -3,8 +3,9 @@
 //
 // Layout: the cases' prepared meshes are concatenated into one set of SoA arrays (global cell and
 // face indices); per-case parameters (scheme, gamma, inlet state, CFL number) and the per-case time
-// step live in small device arrays.  A step is a fixed sequence of persistent kernels (grid = CU
-// count x resident blocks) that pull (case, tile) work items from a device counter: gradient +
+// step live in small device arrays.  A step is a fixed sequence of kernels over (case, tile) work
+// items; all but the patch and fused ones (one block per item) are persistent (grid = CU count x
+// resident blocks) and pull their items from a device counter: gradient +
 // limiter over cell items, fluxes over face items (Roe or AUSM chosen per item's case), gather +
 // stage update over cell items with per-item partial reductions, then one block per case reduces
 // its items' partials into the case's residual norms and next time step.  A whole RK step is
@@ -214,6 +215,52 @@ __global__ __launch_bounds__(NT) void kb_cell(const BArgs<T> a) {
     }
 }
 
+// the flux and update arguments of case cs
+template <typename T>
+__device__ __forceinline__ FluxArgs<T> case_flux(const BArgs<T> &a, int32_t cs) {
+    FluxArgs<T> f = a.f;
+    f.P = a.P[cs];
+    return f;
+}
+template <typename T>
+__device__ __forceinline__ UpdArgs case_update(const BArgs<T> &a, int32_t cs) {
+    UpdArgs u = a.u;
+    u.bad = a.u.bad + cs;
+    u.gamma = a.gam[cs];
+    u.cfl = a.cfl[cs];
+    return u;
+}
+
+// the update of a patch's cell c from its residual r (valid: the lane has a cell) and the item's partials
+template <int NV, bool F32, typename T>
+__device__ __forceinline__ void patch_tail(const BArgs<T> &a, const UpdArgs &u, int it, int64_t c, bool valid, double dt,
+                                           const StageIn<NV> &in, const double (&r)[NV]) {
+    const bool L2 = a.u.l2 != 0, DT = a.u.dtred != 0;
+    double red[NV + 1];
+#pragma unroll
+    for (int k = 0; k < NV; k++) red[k] = 0;
+    red[NV] = INFINITY;
+    if (valid) stage_cell<NV, F32>(u, c, dt, in, r, red, L2, DT);
+    if (L2) {
+        double v[NV];
+#pragma unroll
+        for (int k = 0; k < NV; k++) v[k] = red[k];
+        block_partial<NV, false, BLOCK>(v, a.part_l2 + it, a.n_items);
+    }
+    if (DT) {
+        double v[1] = {red[NV]};
+        block_partial<1, true, BLOCK>(v, a.part_dt + it, 1);
+    }
+}
+
+// The patch and fused kernels take one item per block: their items are all of one size, so there is nothing for a
+// queue to balance, and a loop over items kept the next item's addresses and constants in registers (FP64 triangles:
+// kb_fused 162 registers, 3 waves per SIMD, against 128 and 4; kb_patch 126 against 104).  SSP-RK2 steps of 40 cases of
+// triangles, queue / one item per block: second order, 437,360 cells FP64 109 / 85 us, mixed 112 / 68, 41,600 cells
+// 41 / 33 and 40 / 30; first order, 437,360 cells 91 / 54 and 103 / 45.  16 cases of 48,000 tetrahedra: patch 391 /
+// 337, mixed fused 279 / 211.  The blocks follow each other through the cases, so an XCD keeps a stretch of one in its L2.
+// They zero all the queues' counters.
+
 // patch strategy: one item is one patch (BLOCK consecutive cells of a case, a compact patch in the
 // Hilbert order): its faces solved once into LDS (scheme per case), then sums in slot order and the
 // stage update per cell, as the single-case patch kernel does
@@ -222,69 +269,48 @@ __global__ __launch_bounds__(BLOCK) void kb_patch(const BArgs<T> a, const PatchA
     constexpr int NV = DIM + 2;
     constexpr bool F32 = std::is_same<T, float>::value;
     extern __shared__ double gsh[];  // NV x patch faces, component-major
-    reset_others(a.cnt, a.own);
-    const bool L2 = a.u.l2 != 0, DT = a.u.dtred != 0;
-    for (;;) {
-        const int it = pull(a.cnt, a.own);  // (its barrier also ends the previous item's LDS reads)
-        if (it >= a.n_items) break;
-        const Item I = a.items[it];
-        FluxArgs<T> fa = a.f;
-        fa.P = a.P[I.cs];
-        const bool roe = a.scheme[I.cs] == MST_SCHEME_ROE;
-        const int32_t f0 = p.start[I.pad];
-        const int npf = p.start[I.pad + 1] - f0;
-        for (int i = threadIdx.x; i < npf; i += BLOCK) {
-            int64_t f;
-            int info;
-            patch_face(p, fa.finfo, f0 + i, f, info);
-            const int kind = info & 15;
-            double n64[DIM];
-            T X[NV], Y[NV];
-            face_load<DIM, SECOND, T>(fa, f, kind, n64, X, Y);
-            double g[NV];
-            face_solve<DIM, SCHEME_RUNTIME, T>(fa.P, roe, kind, info >> 4, n64, X, Y, g);
+    reset_others(a.cnt, -1);
+    const int it = (int)block_id();
+    const Item I = a.items[it];
+    const FluxArgs<T> fa = case_flux(a, I.cs);
+    const bool roe = a.scheme[I.cs] == MST_SCHEME_ROE;
+    const int32_t f0 = p.start[I.pad];
+    const int npf = p.start[I.pad + 1] - f0;
+    for (int i = threadIdx.x; i < npf; i += BLOCK) {
+        int64_t f;
+        int info;
+        patch_face(p, fa.finfo, f0 + i, f, info);
+        const int kind = info & 15;
+        double n64[DIM];
+        T X[NV], Y[NV];
+        face_load<DIM, SECOND, T>(fa, f, kind, n64, X, Y);
+        double g[NV];
+        face_solve<DIM, SCHEME_RUNTIME, T>(fa.P, roe, kind, info >> 4, n64, X, Y, g);
 #pragma unroll
-            for (int k = 0; k < NV; k++) gsh[k * npf + i] = g[k];
-        }
-        __syncthreads();
-        UpdArgs ua = a.u;
-        ua.bad = a.u.bad + I.cs;
-        ua.dt = a.dts + I.cs;
-        ua.gamma = a.gam[I.cs];
-        ua.cfl = a.cfl[I.cs];
-        double red[NV + 1];
-#pragma unroll
-        for (int k = 0; k < NV; k++) red[k] = 0;
-        red[NV] = INFINITY;
-        const int64_t c = I.begin + (int)threadIdx.x;
-        if (c < I.end) {
-            int cl[MAXF];
-#pragma unroll
-            for (int s = 0; s < MAXF; s++) cl[s] = p.loc[(int64_t)s * ua.nc + c];
-            double r[NV];
-            patch_sum<NV, MAXF, F32>(gsh, npf, cl, r);
-            stage_cell<NV, F32>(ua, c, ua.dt[0], r, red, L2, DT);
-        }
-        if (L2) {
-            double v[NV];
-#pragma unroll
-            for (int k = 0; k < NV; k++) v[k] = red[k];
-            block_partial<NV, false, BLOCK>(v, a.part_l2 + it, a.n_items);
-        }
-        if (DT) {
-            double v[1] = {red[NV]};
-            block_partial<1, true, BLOCK>(v, a.part_dt + it, 1);
-        }
+        for (int k = 0; k < NV; k++) gsh[k * npf + i] = g[k];
     }
+    const UpdArgs u = case_update(a, I.cs);
+    const int64_t c = I.begin + (int)threadIdx.x;
+    const bool valid = c < I.end;
+    int cl[MAXF];
+#pragma unroll
+    for (int s = 0; s < MAXF; s++) cl[s] = valid ? p.loc[(int64_t)s * u.nc + c] : -1;
+    StageIn<NV> in;
+    if (valid) stage_load<NV, F32>(u, c, in);
+    const double dt = a.dts[I.cs];
+    __syncthreads();
+    double r[NV];
+    patch_sum<NV, MAXF, F32>(gsh, npf, cl, r);
+    patch_tail<NV, F32>(a, u, it, c, valid, dt, in, r);
 }
 
 // fused strategy (order 2): one item is one patch, whose cells' and halo's gradients, face states and
 // fluxes stay in the block (fused_patch), then sums in slot order and the stage update per cell
-// FP32 triangles: 5 resident waves per SIMD (at most 96 VGPRs, 4 registers spilled); elsewhere the
-// compiler chooses.
+// 2D triangles: 4 resident waves per SIMD in FP64 (at most 128 VGPRs, where the compiler would take 133), 5 in FP32;
+// elsewhere the compiler chooses.
 template <int DIM, typename T, int MAXF>
 constexpr int kb_fused_waves() {
-    return (sizeof(T) == 4 && DIM == 2 && MAXF == 3) ? 5 : 1;
+    return DIM == 2 && MAXF == 3 ? (sizeof(T) == 4 ? 5 : 4) : 1;
 }
 
 template <int DIM, int LIM, typename T, int MAXF>
@@ -293,47 +319,26 @@ __global__ __launch_bounds__(BLOCK, (kb_fused_waves<DIM, T, MAXF>())) void kb_fu
     constexpr int NV = DIM + 2;
     constexpr bool F32 = std::is_same<T, float>::value;
     extern __shared__ double sh[];
-    reset_others(a.cnt, a.own);
-    const bool L2 = a.u.l2 != 0, DT = a.u.dtred != 0;
-    for (;;) {
-        const int it = pull(a.cnt, a.own);  // (its barrier also ends the previous item's LDS reads)
-        if (it >= a.n_items) break;
-        const Item I = a.items[it];
-        FluxArgs<T> fa = a.f;
-        fa.P = a.P[I.cs];
-        const bool roe = a.scheme[I.cs] == MST_SCHEME_ROE;
-        const int32_t f0 = p.start[I.pad];
-        FusedLds<T> L(sh, p.start[I.pad + 1] - f0, NV);
-        int cl[MAXF];
-        // (no early fetch of the update's inputs here: with both schemes inlined it would cost a wave)
-        fused_patch<DIM, SCHEME_RUNTIME, LIM, T, MAXF, fused_lds_normals<DIM>()>(a.g, fa, roe, p, h, I.pad, I.begin,
-                                                                                I.end, a.u.nc, f0, L, cl, []() {});
-        UpdArgs ua = a.u;
-        ua.bad = a.u.bad + I.cs;
-        ua.dt = a.dts + I.cs;
-        ua.gamma = a.gam[I.cs];
-        ua.cfl = a.cfl[I.cs];
-        double red[NV + 1];
-#pragma unroll
-        for (int k = 0; k < NV; k++) red[k] = 0;
-        red[NV] = INFINITY;
-        const int64_t c = I.begin + (int)threadIdx.x;
-        if (c < I.end) {
-            double r[NV];
-            patch_sum<NV, MAXF, F32>(L.g, L.npf, cl, r);
-            stage_cell<NV, F32>(ua, c, ua.dt[0], r, red, L2, DT);
-        }
-        if (L2) {
-            double v[NV];
-#pragma unroll
-            for (int k = 0; k < NV; k++) v[k] = red[k];
-            block_partial<NV, false, BLOCK>(v, a.part_l2 + it, a.n_items);
-        }
-        if (DT) {
-            double v[1] = {red[NV]};
-            block_partial<1, true, BLOCK>(v, a.part_dt + it, 1);
-        }
-    }
+    reset_others(a.cnt, -1);
+    const int it = (int)block_id();
+    const Item I = a.items[it];
+    const FluxArgs<T> fa = case_flux(a, I.cs);
+    const bool roe = a.scheme[I.cs] == MST_SCHEME_ROE;
+    const int32_t f0 = p.start[I.pad];
+    FusedLds<T> L(sh, p.start[I.pad + 1] - f0, NV);
+    int cl[MAXF];
+    // (no early fetch of the update's inputs here: 437,360 cells 92 us per step against 85, with both schemes inlined
+    // it costs a wave or spills)
+    fused_patch<DIM, SCHEME_RUNTIME, LIM, T, MAXF, fused_lds_normals<DIM>()>(a.g, fa, roe, p, h, I.pad, I.begin, I.end,
+                                                                            a.u.nc, f0, L, cl, []() {});
+    const UpdArgs u = case_update(a, I.cs);
+    const int64_t c = I.begin + (int)threadIdx.x;
+    const bool valid = c < I.end;
+    StageIn<NV> in;
+    if (valid) stage_load<NV, F32>(u, c, in);
+    double r[NV];
+    patch_sum<NV, MAXF, F32>(L.g, L.npf, cl, r);
+    patch_tail<NV, F32>(a, u, it, c, valid, a.dts[I.cs], in, r);
 }
 
 template <int DIM, typename T, int NT>
@@ -792,27 +797,31 @@ BArgs<T> base_args(const mst_batch *b, int isrc) {
 }
 
 template <typename K>
-int persistent_grid(const mst_batch *b, K kernel, int nt, int n_items, int *grid, size_t shm = 0) {
+int persistent_grid(const mst_batch *b, K kernel, int nt, int n_items, int *grid) {
     int per_cu = 0;
-    HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, nt, shm));
+    HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, nt, 0));
     *grid = std::max(1, std::min(n_items, std::max(per_cu, 1) * b->ncu));
     return MST_OK;
 }
 
 template <typename K, typename... A>
-int launch_persistent_shm(mst_batch *b, K kernel, int nt, size_t shm, int n_items, const A &...args) {
+int launch_persistent(mst_batch *b, K kernel, int nt, int n_items, const A &...args) {
     if (n_items <= 0) return MST_OK;
     int grid = 0;
-    int rc = persistent_grid(b, kernel, nt, n_items, &grid, shm);
+    int rc = persistent_grid(b, kernel, nt, n_items, &grid);
     if (rc) return rc;
-    hipLaunchKernelGGL(kernel, dim3(grid), dim3(nt), (uint32_t)shm, b->stream, args...);
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(nt), 0, b->stream, args...);
     HIPCHK(hipGetLastError());
     return MST_OK;
 }
 
+// one block per item (kb_patch, kb_fused)
 template <typename K, typename... A>
-int launch_persistent(mst_batch *b, K kernel, int nt, int n_items, const A &...args) {
-    return launch_persistent_shm(b, kernel, nt, 0, n_items, args...);
+int launch_items(mst_batch *b, K kernel, size_t shm, int n_items, const A &...args) {
+    if (n_items <= 0) return MST_OK;
+    hipLaunchKernelGGL(kernel, dim3((uint32_t)n_items), dim3(BLOCK), (uint32_t)shm, b->stream, args...);
+    HIPCHK(hipGetLastError());
+    return MST_OK;
 }
 
 template <int DIM, typename T, int NT>
@@ -909,9 +918,9 @@ int run_patch(mst_batch *b, int stage, int is, int in, const Stage &sg, int iout
     pa.loc = b->ploc;
     pa.fi = b->pfi;
     const size_t shm = (size_t)b->max_pf * b->nv * sizeof(double);
-#define MST_BPATCH(MF)                                                                                        \
-    if (b->order >= 2) return launch_persistent_shm(b, kb_patch<DIM, true, T, MF>, BLOCK, shm, a.n_items, a, pa); \
-    return launch_persistent_shm(b, kb_patch<DIM, false, T, MF>, BLOCK, shm, a.n_items, a, pa);
+#define MST_BPATCH(MF)                                                                             \
+    if (b->order >= 2) return launch_items(b, kb_patch<DIM, true, T, MF>, shm, a.n_items, a, pa); \
+    return launch_items(b, kb_patch<DIM, false, T, MF>, shm, a.n_items, a, pa);
     if (b->slots == 3) { MST_BPATCH(3) }
     MST_BPATCH(4)
 #undef MST_BPATCH
@@ -943,7 +952,7 @@ int run_fused(mst_batch *b, int stage, int is, int in, const Stage &sg, int iout
     ha.loc = b->hloc;
     b->hg.args<T>(ha);
     const size_t shm = fused_lds_bytes(DIM, b->nv, b->max_pf, std::is_same<T, float>::value, fused_lds_normals<DIM>());
-#define MST_BFUSED(LM, MF) return launch_persistent_shm(b, kb_fused<DIM, LM, T, MF>, BLOCK, shm, a.n_items, a, pa, ha);
+#define MST_BFUSED(LM, MF) return launch_items(b, kb_fused<DIM, LM, T, MF>, shm, a.n_items, a, pa, ha);
 #define MST_BFUSED_L(MF)                                          \
     if (b->limiter == MST_LIM_NONE) { MST_BFUSED(MST_LIM_NONE, MF) } \
     if (b->limiter == MST_LIM_MINMOD) { MST_BFUSED(MST_LIM_MINMOD, MF) } \
