@@ -17,7 +17,8 @@
 //   k_lu_sweep   one lane per cell of one colour; forward: r_f of the cell's faces, D, and
 //                dQ* = (-R - sum_L ...) / D; backward: dQ = dQ* - sum_U ... / D, Q_new = Q + dQ
 //                (and the admissibility check)
-// Both sweeps are memory-bound gathers over the neighbours of a cell, like the residual's gather.
+// Both sweeps are gathers over the neighbours of a cell, like the residual's gather; a colour of a few hundred thousand
+// cells is two or three waves per SIMD, all in step, so they are bound by their loads' latency and then the solves'.
 #pragma once
 #include "kernels.hpp"
 
@@ -175,7 +176,7 @@ __device__ __forceinline__ void lu_offdiag(const double *q, const double *qp, co
 // One cell's sweep (position t, cell c).  P, roe: of the cell's case.
 // (Solving each face once, its flux and radius stored by the lower colour's sweep for the higher's, cut colour 1's
 // vector instructions from 1,770 to 560 per wave and its time from 18.6 to 17.3 us on 300,000 triangles, but colour
-// 0's kernel grew from 22.7 to 24.5 us with the stores: the sweeps are bound by their bytes.  Not kept.)
+// 0's kernel grew from 22.7 to 24.5 us with the stores, and colour 1 waits for its loads either way.  Not kept.)
 template <int DIM, bool FWD, bool LAST, int MAXF, int RSCHEME>
 __device__ __forceinline__ void lu_cell(const LuArgs &a, const Params<double> &P, const bool roe, const int64_t t,
                                         const int64_t c) {
