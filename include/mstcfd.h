@@ -72,8 +72,10 @@ typedef struct {
     double cfl;            /* > 0: mst_step computes dt = cfl * min V / sum (|u_d|+a) S_d; 0: use mst_set_dt */
     double q_inlet[5];     /* inlet ghost state (dim+2 used) */
     /* NEW viscous terms (the intent of RhoSolver::updateViscid, rhoSolver/RhoSolver.cpp:371-429; the
-     * reference runs inviscid, FLAGVISCID 0): mu = kappa = 0 is inviscid.  Viscous runs use the face
-     * strategy and FP64 or mixed single contexts (not batches). */
+     * reference runs inviscid, FLAGVISCID 0): mu = kappa = 0 is inviscid.  Viscous runs need
+     * a single context (not a batch), FP64 or mixed.  With MST_STRATEGY_FACE, on meshes without patch tables and on
+     * meshes with faces of unknown type their stages run the face kernels, else the patch kernels (the same bits);
+     * mst_get_face_flux and mst_residual_update then form the last stage's face fluxes when asked. */
     double mu;             /* dynamic viscosity (include/CONST.h:46: 1.7894e-5) */
     double lam;            /* bulk coefficient (CONST.h:47: -0.666667 mu) */
     double kappa;          /* thermal conductivity (CONST.h:48 TEMPK: 0.0242) */
@@ -289,7 +291,8 @@ int mst_monitor_maxrel_noalloc(const double *qnew, const double *qold, int64_t n
 /* ---------------------------------------------------------------- inspection (tests) */
 /* residual R_i = sum_f sum_d n_out,d F_f[:,d] (rhoSolver/RhoSolver.cpp:51-55) of the Old state, file order */
 int mst_get_residual(mst_ctx *ctx, double *R, int64_t n_cells);
-/* per-face G_f of the last mst_face_flux, file order, n_faces*nv */
+/* per-face G_f of the last mst_face_flux (or mst_get_residual, stage of MST_STRATEGY_FACE, or stage of a viscous
+ * configuration), file order, n_faces*nv */
 int mst_get_face_flux(mst_ctx *ctx, double *G, int64_t n_faces);
 /* gradient (n_cells*nv*dim) and limiter factor (n_cells*nv) of the Old state, file order */
 int mst_get_gradient(mst_ctx *ctx, double *grad, double *phi, int64_t n_cells);
@@ -406,7 +409,8 @@ int mst_ctx_warm_start(mst_ctx *ctx, mst_mlp *m, const double *cond, int n_cond)
 #define MST_K_PATCH 5 /* patch fluxes in LDS + gather + update (MST_STRATEGY_PATCH) */
 #define MST_K_FUSED 6 /* gradients + face states + fluxes in LDS + gather + update (MST_STRATEGY_FUSED) */
 #define MST_K_LUSGS 7 /* LU-SGS colour sweeps (mst_lusgs_step); algorithmic bytes: per launch, averaged */
-#define MST_K_VISC 8 /* viscous gradient + face kernels (mu or kappa > 0); algorithmic bytes: per launch, averaged */
+#define MST_K_VISC 8 /* viscous gradient + face kernels of the face route, else the viscous gradients that MST_K_GRAD does not
+                        form (order 1, mixed) (mu or kappa > 0); algorithmic bytes: per launch, averaged */
 #define MST_K_COUNT 9
 /* on: 0 off, 1 events on every launch, n > 1 on one launch in n of each kernel class (counted from
    this call; a timed dispatch costs a few microseconds of throughput) */

@@ -101,6 +101,7 @@ struct mst_ctx {
     Transfer link;            // host states in file order
     bool viscous = false;     // mu or kappa > 0: the viscous kernels (viscous.hpp), patch or face route
     bool visc_patch = false;  // the mesh allows the patch route
+    int g_of = -1;            // the state whose face fluxes G stands for but does not hold yet (ensure_fluxes), or -1
     double *gw = nullptr;     // viscous: per cell Green-Gauss gradients of (u, T), [nc][dim + 1][dim]
     // LU-SGS steady driver (built on first use): cell colours, the cells of each colour in ascending
     // order (colour k: lu_cells[lu_start[k] .. lu_start[k + 1])), face spectral radii, the update

@@ -126,6 +126,7 @@ int run_grad_visc(mst_ctx *x, int isrc) {
 // residual evaluation up to the face fluxes: gradient + limiter (order 2), the flux kernel, and the
 // viscous terms when the configuration has them
 int run_face_flux(mst_ctx *x, int isrc) {
+    x->g_of = -1;
     int rc = ensure_shadow(x, isrc);
     if (rc) return rc;
     if (x->cfg.order >= 2) {
@@ -139,6 +140,11 @@ int run_face_flux(mst_ctx *x, int isrc) {
     if (rc || !x->viscous) return rc;
     return run_viscous(x, isrc);
 }
+
+// G of the last viscous stage, before G is read or its state or configuration replaced.  The patch route of a viscous
+// stage stores no face fluxes, and a viscous context's G is its last stage's whichever route that took: so the
+// stage leaves its state's index and the fluxes are formed here, for the few calls that need them.
+int ensure_fluxes(mst_ctx *x) { return x->g_of < 0 ? (int)MST_OK : run_face_flux(x, x->g_of); }
 
 template <int NV, bool GT>
 int run_update_t(mst_ctx *x, int mode, int is, int in, const Stage &sg, int iout) {
@@ -218,6 +224,7 @@ int run_stage(mst_ctx *x, int mode, int is, int in, const Stage &sg, int iout) {
             rc = x->dim == 2 ? run_patch_t<2, double>(x, mode, is, in, sg, iout)
                              : run_patch_t<3, double>(x, mode, is, in, sg, iout);
         if (rc == MST_OK && iout >= 0) x->shadow_ok[iout] = x->mixed;
+        x->g_of = is;
         return rc;
     }
     if (x->resolved == MST_STRATEGY_FUSED) {
@@ -1018,6 +1025,8 @@ int mst_ctx_set_config(mst_ctx *ctx, const mst_config *cfg) {
     CTX_GUARD(ctx);
     int rc = check_config(cfg);
     if (rc) return rc;
+    rc = ensure_fluxes(ctx);
+    if (rc) return rc;
     HIPCHK(hipStreamSynchronize(ctx->stream));
     ctx->cfg = *cfg;
     ctx->dt_valid = false;
@@ -1030,6 +1039,10 @@ const mst_prep *mst_ctx_prep(const mst_ctx *ctx) { return ctx ? &ctx->prep : nul
 int mst_set_state(mst_ctx *ctx, const double *Q, int64_t n_cells) {
     CTX_GUARD(ctx);
     if (!Q || n_cells != ctx->nc) return mst::fail(MST_E_ARG, "state size does not match the mesh");
+    if (ctx->g_of == ctx->iold) {
+        int rc = ensure_fluxes(ctx);
+        if (rc) return rc;
+    }
     HIPCHK(ctx->link.put(ctx->stream, ctx->nc, ctx->nv, ctx->cnew, Q, &ctx->Q[ctx->iold], 1));
     ctx->shadow_ok[ctx->iold] = false;
     ctx->dt_valid = false;
@@ -1064,7 +1077,9 @@ int mst_face_flux(mst_ctx *ctx) {
 
 int mst_residual_update(mst_ctx *ctx) {
     CTX_GUARD(ctx);
-    int rc = run_update(ctx, UPD_STAGE | UPD_CHECK, ctx->iold, ctx->iold, Stage{}, ctx->inew);
+    int rc = ensure_fluxes(ctx);
+    if (rc) return rc;
+    rc = run_update(ctx, UPD_STAGE | UPD_CHECK, ctx->iold, ctx->iold, Stage{}, ctx->inew);
     if (rc) return rc;
     return check_bad(ctx);
 }
@@ -1333,6 +1348,10 @@ int mst_ctx_warm_start(mst_ctx *ctx, mst_mlp *mlp, const double *cond, int n_con
     if (n_in != ctx->dim + n_cond || n_out != ctx->nv)
         return mst::fail(MST_E_ARG, "network sizes do not match (dim + conditions) -> nv");
     if (!(cond[0] > 0)) return mst::fail(MST_E_ARG, "the first condition (freestream Mach number) must be positive");
+    if (ctx->g_of != ctx->inew) {  // (every other buffer is written here)
+        int rc = ensure_fluxes(ctx);
+        if (rc) return rc;
+    }
     WarmArgs w;
     w.nc = ctx->nc;
     w.cxc = ctx->cxc;
@@ -1383,6 +1402,8 @@ int mst_get_residual(mst_ctx *ctx, double *R, int64_t n_cells) {
 int mst_get_face_flux(mst_ctx *ctx, double *G, int64_t n_faces) {
     CTX_GUARD(ctx);
     if (!G || n_faces != ctx->nf) return mst::fail(MST_E_ARG, "size does not match the mesh");
+    int rc = ensure_fluxes(ctx);
+    if (rc) return rc;
     const int nv = ctx->nv;
     std::vector<double> buf(ctx->nf * nv);
     HIPCHK(hipStreamSynchronize(ctx->stream));
