@@ -1562,21 +1562,29 @@ __global__ __launch_bounds__(FIN) void k_finish_min(const double *__restrict__ s
     }
 }
 
-// The W maxima of k_maxrel's partials (all >= 0, no NaN: any order) to the host's board in one block.  28 partials: 4 us
-// where k_finish takes 8 and a stream synchronisation and a copy followed.
-template <int W>
-__global__ __launch_bounds__(BLOCK) void k_finish_max(const double *__restrict__ part, int64_t n, Board *__restrict__ b,
-                                                      uint32_t seq) {
-    __shared__ double s[W][BLOCK / 64];
+// The W maxima of k_maxrel's partials (all >= 0, no NaN: any order) to the host's board in one block of NT lanes, eight
+// loads per field of each lane in flight together: n <= 8 NT is one round of the memory's latency, so MONITOR_GRID bounds
+// k_maxrel's partials by 8 FIN.  28 partials: 4 us where k_finish takes 8 and a stream synchronisation and a copy followed;
+// the whole call on 2M / 8M / 24.5M triangles: 35 / 113 / 287 us (41 / 143 / 440 with 256 lanes of one load each).
+constexpr int64_t MONITOR_GRID = 8 * FIN;
+template <int W, int NT>
+__global__ __launch_bounds__(NT) void k_finish_max(const double *__restrict__ part, int64_t n, Board *__restrict__ b,
+                                                   uint32_t seq) {
+    __shared__ double s[W][NT / 64];
     double v[W];
 #pragma unroll
     for (int k = 0; k < W; k++) v[k] = 0;
-    for (int64_t i = threadIdx.x; i < n; i += BLOCK) {
+    for (int64_t i = threadIdx.x; i < n; i += 8 * NT) {
+        double x[W][8];
 #pragma unroll
-        for (int k = 0; k < W; k++) {
-            const double x = part[k * n + i];
-            if (v[k] < x) v[k] = x;
-        }
+        for (int k = 0; k < W; k++)
+#pragma unroll
+            for (int u = 0; u < 8; u++) x[k][u] = i + u * NT < n ? part[k * n + i + u * NT] : 0;
+#pragma unroll
+        for (int k = 0; k < W; k++)
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+                if (v[k] < x[k][u]) v[k] = x[k][u];
     }
 #pragma unroll
     for (int k = 0; k < W; k++) {
@@ -1589,7 +1597,7 @@ __global__ __launch_bounds__(BLOCK) void k_finish_max(const double *__restrict__
     __syncthreads();
     if ((int)threadIdx.x < W) {
         double m = s[threadIdx.x][0];
-        for (int w = 1; w < BLOCK / 64; w++)
+        for (int w = 1; w < NT / 64; w++)
             if (m < s[threadIdx.x][w]) m = s[threadIdx.x][w];
         b->mon[threadIdx.x] = m;
         __threadfence_system();

@@ -608,6 +608,24 @@ int fetch_cells(mst_ctx *x, const double *dsrc, int width, double *out) {
     return MST_OK;
 }
 
+// max |new - old| / old per field
+template <int NV>
+int run_monitor(mst_ctx *x, double *out) {
+    const int64_t n = std::min(x->nblk_c, MONITOR_GRID);
+    int rc = launch(x, -1, k_maxrel<NV>, n * BLOCK, x->nc, (const double *)x->Q[x->inew], (const double *)x->Q[x->iold],
+                    x->part);
+    if (rc) return rc;
+    const uint32_t seq = ++x->board_seq;
+    if (n <= 8 * BLOCK)
+        hipLaunchKernelGGL((k_finish_max<NV, BLOCK>), dim3(1), dim3(BLOCK), 0, x->stream, (const double *)x->part, n, x->board, seq);
+    else
+        hipLaunchKernelGGL((k_finish_max<NV, FIN>), dim3(1), dim3(FIN), 0, x->stream, (const double *)x->part, n, x->board, seq);
+    HIPCHK(hipGetLastError());
+    HIPCHK(board_wait(x->board, seq, x->stream));
+    for (int k = 0; k < NV; k++) out[k] = x->board->mon[k];
+    return MST_OK;
+}
+
 // scal and the bad flag on the board, after the stream's earlier work
 int report(mst_ctx *x, bool take_bad) {
     hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, x->stream, (const double *)x->scal, x->bad, (int)take_bad, x->board,
@@ -1288,22 +1306,7 @@ int mst_residual_norms(mst_ctx *ctx, double *out) {
 int mst_monitor_maxrel(mst_ctx *ctx, double *out) {
     CTX_GUARD(ctx);
     if (!out) return mst::fail(MST_E_ARG, "null argument");
-    int rc = ctx->nv == 4 ? launch(ctx, -1, k_maxrel<4>, ctx->nc, ctx->nc, (const double *)ctx->Q[ctx->inew],
-                                   (const double *)ctx->Q[ctx->iold], ctx->part)
-                          : launch(ctx, -1, k_maxrel<5>, ctx->nc, ctx->nc, (const double *)ctx->Q[ctx->inew],
-                                   (const double *)ctx->Q[ctx->iold], ctx->part);
-    if (rc) return rc;
-    const uint32_t seq = ++ctx->board_seq;
-    if (ctx->nv == 4)
-        hipLaunchKernelGGL(k_finish_max<4>, dim3(1), dim3(BLOCK), 0, ctx->stream, (const double *)ctx->part, ctx->nblk_c,
-                           ctx->board, seq);
-    else
-        hipLaunchKernelGGL(k_finish_max<5>, dim3(1), dim3(BLOCK), 0, ctx->stream, (const double *)ctx->part, ctx->nblk_c,
-                           ctx->board, seq);
-    HIPCHK(hipGetLastError());
-    HIPCHK(board_wait(ctx->board, seq, ctx->stream));
-    for (int k = 0; k < ctx->nv; k++) out[k] = ctx->board->mon[k];
-    return MST_OK;
+    return ctx->nv == 4 ? run_monitor<4>(ctx, out) : run_monitor<5>(ctx, out);
 }
 
 int mst_monitor_maxrel_noalloc(const double *qnew, const double *qold, int64_t n_cells, int nv, double *out,
