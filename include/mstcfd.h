@@ -235,8 +235,9 @@ int mst_step(mst_ctx *ctx, int nsteps);
  * otherwise).  FUSED (order 2; order 1 runs PATCH): the patch kernel also computes the limited
  * gradients of its cells and of its halo and keeps the face states in LDS, one kernel per stage.
  * All give the same result bit for bit.  AUTO (default): the first stage after creation
- * or a configuration change times one stage of each available strategy on the context's own mesh
- * and keeps the fastest; mst_get_strategy then reports it.  mst_face_flux / mst_residual_update keep
+ * or a configuration change times a few stages of each strategy that may be the fastest on the context's
+ * own mesh (up to 512 blocks of cells: patch and fused, where available) and keeps the fastest;
+ * mst_get_strategy then reports it.  mst_face_flux / mst_residual_update keep
  * the face split whatever the strategy. */
 #define MST_STRATEGY_FACE 0
 #define MST_STRATEGY_CELL 1

@@ -834,58 +834,83 @@ int lu_inline_iterations(mst_ctx *x, int n) {
 }
 
 
-// AUTO: time one stage of each strategy on this mesh and configuration (outputs go to a spare state
-// buffer; the Old and New states are untouched) and keep the faster
+// x->resolved = the fastest of the n candidates: REPS stages of each are timed in each round, outputs to a spare state
+// buffer (the Old and New states are untouched).  Stages of a few microseconds: the rounds are queued behind each
+// other and the better one counts.  (Three stages from an empty queue, 12 us of launches, picked an 8.5 us kernel over a
+// 5.6 us one about every other time.)
+int time_strategies(mst_ctx *x, const int *cand, int n, int rounds) {
+    constexpr int REPS = 3;
+    int spare = 0;
+    while (spare == x->iold || spare == x->inew) spare++;
+    const bool timing = x->timing;
+    x->timing = false;
+    hipEvent_t ev[16] = {};
+    hipError_t e = hipSuccess;
+    int rc = MST_OK;
+    for (int k = 0; k < 2 * rounds * n && e == hipSuccess; k++) e = hipEventCreate(&ev[k]);
+    for (int k = 0; k < rounds * n && !rc && e == hipSuccess; k++) {
+        x->resolved = cand[k % n];
+        if (k < n) rc = run_stage(x, UPD_STAGE, x->iold, x->iold, Stage{}, spare);  // warm-up
+        if (!rc) e = hipEventRecord(ev[2 * k], x->stream);
+        for (int r = 0; r < REPS && !rc; r++) rc = run_stage(x, UPD_STAGE, x->iold, x->iold, Stage{}, spare);
+        if (!rc && e == hipSuccess) e = hipEventRecord(ev[2 * k + 1], x->stream);
+    }
+    x->timing = timing;
+    // waits for the trials; they may have flagged their (unchecked) outputs, e.g. with no time step set yet
+    if (!rc) rc = report(x, true);
+    if (!rc && e == hipSuccess) e = hipEventSynchronize(ev[2 * rounds * n - 1]);
+    float best = INFINITY;
+    x->resolved = cand[0];
+    for (int k = 0; k < rounds * n && !rc && e == hipSuccess; k++) {
+        float ms = 0;
+        if (hipEventElapsedTime(&ms, ev[2 * k], ev[2 * k + 1]) == hipSuccess && ms < best) {
+            best = ms;
+            x->resolved = cand[k % n];
+        }
+    }
+    for (hipEvent_t v : ev)
+        if (v) (void)hipEventDestroy(v);
+    HIPCHK(e);
+    return rc;
+}
+
+// Blocks up to which AUTO looks no further than the patch kernels, where a mesh has patch tables.  On 20 meshes of 2 to
+// 131,072 triangles, quadrilaterals and tetrahedra, both orders, schemes and precisions, viscous or not, a stage of the
+// face or the cell strategy took 1.03 to 1.65 times the better of patch and fused (mixed 3D AUSM on 10,368 cells: the
+// same, 14.7 us); at 140,000 to 162,000 cells 1.06 to 1.37.  So a first step of order 1 costs no trial there, and one
+// of order 2 14 stages: about 150 to 250 us, where timing all four strategies well enough took 600 to 1,500.
+constexpr int64_t AUTO_PATCH_MAX = 512;
+
+// AUTO: the strategy for this mesh and configuration.  Where more than one can be the fastest, a few stages of each are
+// timed (outputs go to a spare state buffer; the Old and New states are untouched).
 int resolve_strategy(mst_ctx *x) {
     if (x->strategy != MST_STRATEGY_AUTO) {
         x->resolved = x->strategy;
         return MST_OK;
     }
-    int spare = 0;
-    while (spare == x->iold || spare == x->inew) spare++;
-    const bool timing = x->timing;
-    x->timing = false;
-    hipEvent_t e0 = nullptr, e1 = nullptr;
-    HIPCHK(hipEventCreate(&e0));
-    HIPCHK(hipEventCreate(&e1));
-    float best = INFINITY;
-    int pick = MST_STRATEGY_FACE, rc = MST_OK;
-    // Stages of a few microseconds: the queue is filled ahead of the first event and the better of two rounds of more
-    // stages counts; three stages from an empty queue (12 us of launches) picked the 8.5 us cell kernel over the
-    // 5.6 us patch kernel about every other time on 7,000 cells.
-    const bool few = x->nblk_c <= 512;
-    const int lead = few ? 3 : 1, reps = few ? 8 : 3;
-    const int all[] = {MST_STRATEGY_FACE, MST_STRATEGY_CELL, MST_STRATEGY_PATCH, MST_STRATEGY_FUSED};
-    for (int k = 0; k < (few ? 8 : 4) && !rc; k++) {
-        const int s = all[k & 3];
-        if ((s == MST_STRATEGY_PATCH || s == MST_STRATEGY_FUSED) && !x->patch_ok) continue;
-        if (s == MST_STRATEGY_FUSED && !x->fused_ok) continue;
-        // viscous stages have two routes: the face strategy's, and the patch route under any other
-        if (x->viscous && s != MST_STRATEGY_FACE && s != (x->patch_ok ? MST_STRATEGY_PATCH : MST_STRATEGY_CELL)) continue;
-        x->resolved = s;
-        for (int r = 0; r < lead && !rc; r++) rc = run_stage(x, UPD_STAGE, x->iold, x->iold, Stage{}, spare);  // warm-up
-        if (rc) break;
-        if (hipEventRecord(e0, x->stream) != hipSuccess) break;
-        for (int r = 0; r < reps && !rc; r++) rc = run_stage(x, UPD_STAGE, x->iold, x->iold, Stage{}, spare);
-        if (rc || hipEventRecord(e1, x->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess) break;
-        float ms = 0;
-        if (hipEventElapsedTime(&ms, e0, e1) == hipSuccess && ms < best) {
-            best = ms;
-            pick = s;
+    const bool few = x->patch_ok && x->nblk_c <= AUTO_PATCH_MAX;
+    int cand[4], n = 0;
+    if (x->viscous) {  // two routes: the face strategy's, and the patch route under any other
+        if (!few || !x->visc_patch) cand[n++] = MST_STRATEGY_FACE;
+        if (x->visc_patch) cand[n++] = MST_STRATEGY_PATCH;
+    } else {
+        if (!few) {
+            cand[n++] = MST_STRATEGY_FACE;
+            cand[n++] = MST_STRATEGY_CELL;
         }
+        if (x->patch_ok) cand[n++] = MST_STRATEGY_PATCH;
+        if (x->fused_ok && x->cfg.order >= 2) cand[n++] = MST_STRATEGY_FUSED;  // (order 1: the patch kernel)
     }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    x->timing = timing;
-    x->resolved = pick;
-    // the trial stages may have flagged their (unchecked) outputs, e.g. with no time step set yet
-    HIPCHK(hipStreamSynchronize(x->stream));
-    HIPCHK(hipMemset(x->bad, 0, sizeof(int)));
-    if (pick != MST_STRATEGY_FUSED) {  // the fused trial's halo copy (0.64 N_c entries in 3D) is not kept
+    x->resolved = cand[0];
+    if (n > 1) {
+        const int rc = time_strategies(x, cand, n, few ? 2 : 1);
+        if (rc) return rc;
+    }
+    if (x->resolved != MST_STRATEGY_FUSED) {  // the fused kernel's halo copy (0.64 N_c entries in 3D) is not kept
         x->hg.release();
         x->hg_dirty = true;
     }
-    return rc;
+    return MST_OK;
 }
 
 }  // namespace
