@@ -25,6 +25,9 @@ using namespace mstk;
             return mst::fail(MST_E_HIP, std::string(#expr) + ": " + hipGetErrorString(_e));              \
     } while (0)
 
+// blocks of BLOCK cells up to which patches are of SUB_PATCH cells, 2D and 3D (mst_ctx::patch_cells)
+constexpr int64_t SUB_PATCH_MAX[2] = {128, 64};
+
 // ====================================================================================== context
 struct mst_ctx {
     mst_prep prep;
@@ -91,6 +94,7 @@ struct mst_ctx {
     // 18.8 (95), 20.6 / 20.2 (133); first order 2D 11.4 / 9.9 (32), 11.8 / 11.7 (113), 12.0 / 13.2 (133); viscous 2D
     // 24.6 / 22.8 (32), 26.5 / 25.9 (113), 26.9 / 28.2 (133); patch 3D 31.2 / 29.2 (32), 31.6 / 29.8 (52), 32.4 /
     // 32.7 (80); first order 3D 17.0 / 15.8 (52), 17.1 / 17.7 (65); the mixed form in 3D 28.7 / 29.3 (24), so not there.
+    // (A configuration of the other precision rebuilds the tables.)
     int patch_cells = BLOCK;  // BLOCK or SUB_PATCH
     int64_t n_patch = 0;
     int64_t dt_cnt[2] = {0, 0}, l2_cnt = 0;  // partials in pdt[i] and part, as their last writer left them
@@ -273,6 +277,12 @@ inline ViscArgs visc_args(const mst_ctx *x, int isrc) {
     a.kappa = x->cfg.kappa;
     a.cv = x->cfg.cv;
     return a;
+}
+
+// whether kernels of dimension DIM and arithmetic T ever have patches of SUB_PATCH cells (patch_cells in solver.hip)
+template <int DIM, typename T>
+constexpr bool has_sub_patches() {
+    return DIM == 2 || std::is_same<T, double>::value;
 }
 
 // one stage (mode includes UPD_STAGE) with the patch strategy (its gradient kernel has run) or the fused one;

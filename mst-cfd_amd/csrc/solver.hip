@@ -395,14 +395,30 @@ int build_incidence(mst_ctx *x) {
     return rc;
 }
 
+// cells per patch of the current configuration (the sweeps stand at mst_ctx::patch_cells)
+int patch_cells(const mst_ctx *x) {
+    const bool sub = x->nblk_c <= SUB_PATCH_MAX[x->dim - 2] && (x->dim == 2 || x->cfg.precision != MST_PREC_MIXED);
+    return sub ? SUB_PATCH : BLOCK;
+}
+
 // Patch tables: for each patch of patch_cells consecutive cells, the faces that carry a flux into one of its
 // cells (ascending; a face joining two of its cells once), and for each cell slot (local index << 1) |
 // is_c1, or -1 for an empty slot or a zero-flux face; and each patch's halo for the fused kernel.
 // The kernels keep a patch's face states and fluxes in LDS, so the strategies need at most 4 slots and
 // 16 * NV bytes per face of the largest patch within 64 KiB.
+// Built at creation, and again by a configuration whose patches have another size.
 int build_patches(mst_ctx *x) {
     const mst::Prepared &P = x->prep.P;
     x->patch_ok = x->fused_ok = false;
+    for (void **b : {(void **)&x->pstart, (void **)&x->pface, (void **)&x->pfi, (void **)&x->ploc, (void **)&x->hstart,
+                     (void **)&x->hcell, (void **)&x->hloc}) {
+        if (*b) (void)hipFree(*b);
+        *b = nullptr;
+    }
+    x->hg.release();
+    x->hg_dirty = true;
+    x->patch_cells = patch_cells(x);
+    x->n_patch = (x->nc + x->patch_cells - 1) / x->patch_cells;
     if (x->slots > 4) return MST_OK;
     const int64_t nc = x->nc, pc = x->patch_cells, nb = x->n_patch;
     std::vector<int32_t> start(nb + 1, 0), face, list, hstart(nb + 1, 0), hcell, halo;
@@ -986,9 +1002,6 @@ int mst_ctx_create(const mst_mesh *m, const mst_config *cfg, mst_ctx **out) {
     x->nblk_f = (x->nf + BLOCK - 1) / BLOCK;
     x->wide_patch = x->nblk_c <= (x->dim == 3 ? 512 : 256);
     x->wide_fused = x->nblk_c <= (x->dim == 2 ? 512 : 256);
-    x->patch_cells = x->nblk_c <= (x->dim == 2 ? 128 : 64) && (x->dim == 2 || cfg->precision != MST_PREC_MIXED) ? SUB_PATCH
-                                                                                                           : BLOCK;
-    x->n_patch = (x->nc + x->patch_cells - 1) / x->patch_cells;
 #define TRY(e)            \
     do {                  \
         int _r = (e);     \
@@ -1035,8 +1048,10 @@ int mst_ctx_create(const mst_mesh *m, const mst_config *cfg, mst_ctx **out) {
     TRY(dalloc(&x->G, x->nf * x->nv));
     TRY(dalloc(&x->rec, (int64_t)x->slots * x->nc * x->nv));
     TRY(dalloc(&x->scal, 16));
-    TRY(dalloc(&x->part, std::max(x->n_patch + x->nblk_c, x->nblk_f) * x->nv + 16));
-    for (int i = 0; i < 2; i++) TRY(dalloc(&x->pdt[i], std::max(x->n_patch, x->nblk_c)));
+    // (a configuration may change the size of the patches)
+    const int64_t most = x->nblk_c <= SUB_PATCH_MAX[x->dim - 2] ? (x->nc + SUB_PATCH - 1) / SUB_PATCH : x->nblk_c;
+    TRY(dalloc(&x->part, std::max(most + x->nblk_c, x->nblk_f) * x->nv + 16));
+    for (int i = 0; i < 2; i++) TRY(dalloc(&x->pdt[i], most));
     TRY(dalloc(&x->fin_mid, 12 * (x->nblk_c / FIN_CHUNK + 2)));
     TRY(dalloc(&x->bad, 1));
     if (hipHostMalloc((void **)&x->board, sizeof(Board), hipHostMallocCoherent) != hipSuccess) {
@@ -1074,6 +1089,10 @@ int mst_ctx_set_config(mst_ctx *ctx, const mst_config *cfg) {
     ctx->cfg = *cfg;
     ctx->dt_valid = false;
     if (ctx->strategy == MST_STRATEGY_AUTO) ctx->resolved = -1;  // the best strategy depends on the configuration
+    if (ctx->patch_ok && patch_cells(ctx) != ctx->patch_cells) {
+        rc = build_patches(ctx);
+        if (rc) return rc;
+    }
     return upload_config(ctx);
 }
 

@@ -44,7 +44,7 @@ int run_fused_t(mst_ctx *x, int mode, int is, int in, const Stage &sg, int iout)
     const bool roe = x->cfg.scheme == MST_SCHEME_ROE;
     const int lim = x->cfg.limiter;
 #define MST_FUSED_L(SC, LM, MF)                                                                                         \
-    if (x->patch_cells == SUB_PATCH)                                                                                    \
+    if constexpr (has_sub_patches<DIM, T>()) if (x->patch_cells == SUB_PATCH)                                           \
         return launch_patch(x, MST_K_FUSED, k_fused<DIM, SC, LM, T, MF, SUB_PATCH, 2 * SUB_PATCH>, 2 * SUB_PATCH, shm,  \
                             ga, fa, a, pa, ha);                                                                         \
     return x->wide_fused ? launch_patch(x, MST_K_FUSED, k_fused<DIM, SC, LM, T, MF, BLOCK, 2 * BLOCK>, 2 * BLOCK, shm,  \

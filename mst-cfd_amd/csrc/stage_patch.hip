@@ -18,6 +18,7 @@ int run_patch_t(mst_ctx *x, int mode, int is, int in, const Stage &sg, int iout)
     const size_t shm = (size_t)x->max_pf * x->nv * sizeof(double);
     const bool second = x->cfg.order >= 2;
     const bool roe = x->cfg.scheme == MST_SCHEME_ROE, sub = x->patch_cells == SUB_PATCH;
+    constexpr bool SUB = has_sub_patches<DIM, T>();
     if (x->viscous) {
         const ViscFace<DIM> vf{visc_args(x, is)};
 #define MST_PATCH_V_N(MF, SECOND, PC, NT)                                                                                    \
@@ -26,7 +27,7 @@ int run_patch_t(mst_ctx *x, int mode, int is, int in, const Stage &sg, int iout)
                : launch_patch(x, MST_K_PATCH, k_patch<DIM, MST_SCHEME_AUSM, SECOND, T, MF, true, PC, NT, ViscFace<DIM>>, NT, \
                               shm, fa, a, pa, vf);
 #define MST_PATCH_V(MF, SECOND)                      \
-    if (sub) { MST_PATCH_V_N(MF, SECOND, SUB_PATCH, 2 * SUB_PATCH) } \
+    if constexpr (SUB) if (sub) { MST_PATCH_V_N(MF, SECOND, SUB_PATCH, 2 * SUB_PATCH) } \
     if (x->wide_patch) { MST_PATCH_V_N(MF, SECOND, BLOCK, 2 * BLOCK) } \
     MST_PATCH_V_N(MF, SECOND, BLOCK, BLOCK)
         if (x->slots == 3) {
@@ -48,7 +49,7 @@ int run_patch_t(mst_ctx *x, int mode, int is, int in, const Stage &sg, int iout)
     return roe ? launch_patch(x, MST_K_PATCH, k_patch_rec<DIM, MST_SCHEME_ROE, MF, PC, NT>, NT, shm, fa, a, pa, ha)      \
                : launch_patch(x, MST_K_PATCH, k_patch_rec<DIM, MST_SCHEME_AUSM, MF, PC, NT>, NT, shm, fa, a, pa, ha);
 #define MST_PATCH_REC(MF)                      \
-    if (sub) { MST_PATCH_REC_N(MF, SUB_PATCH, 2 * SUB_PATCH) } \
+    if constexpr (SUB) if (sub) { MST_PATCH_REC_N(MF, SUB_PATCH, 2 * SUB_PATCH) } \
     if (x->wide_patch) { MST_PATCH_REC_N(MF, BLOCK, 2 * BLOCK) } \
     MST_PATCH_REC_N(MF, BLOCK, BLOCK)
             if (x->slots == 3) { MST_PATCH_REC(3) }
@@ -66,7 +67,7 @@ int run_patch_t(mst_ctx *x, int mode, int is, int in, const Stage &sg, int iout)
     if (second) { MST_PATCH_N(MF, true, PC, NT) }    \
     MST_PATCH_N(MF, false, PC, NT)
 #define MST_PATCH(MF)                                         \
-    if (sub) { MST_PATCH_W(MF, SUB_PATCH, 2 * SUB_PATCH) }    \
+    if constexpr (SUB) if (sub) { MST_PATCH_W(MF, SUB_PATCH, 2 * SUB_PATCH) }    \
     if (x->wide_patch) { MST_PATCH_W(MF, BLOCK, 2 * BLOCK) }  \
     MST_PATCH_W(MF, BLOCK, BLOCK)
     if (x->slots == 3) { MST_PATCH(3) }
