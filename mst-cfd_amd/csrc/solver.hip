@@ -680,14 +680,24 @@ int build_colours(mst_ctx *x) {
     const int64_t slots = x->slots;
     std::vector<int32_t> nb(slots * nc, -2), fcode(slots * nc, -1);
     std::vector<double> nrm(slots * nc * dim, 0.0);
+    std::vector<LuCount> count(ncol);
+    std::vector<int32_t> seen(nc, -1);  // the colour that last counted the cell as a neighbour
     for (int64_t t = 0; t < nc; t++) {
         const int64_t c = cells[t];
+        LuCount &cnt = count[col[c]];
+        cnt.n++;
         for (int s = 0; s < P.maxf; s++) {
             const int32_t e = P.ell[(int64_t)s * nc + c];
             if (e < 0) break;
             const int32_t f = e >> 1;
             const bool c1side = e & 1;
             const int32_t o = c1side ? P.fc0[f] : P.fc1[f];
+            cnt.inc++;
+            if (o >= 0 && col[o] > col[c]) cnt.inc_hi++;
+            if (o >= 0 && col[o] != col[c] && seen[o] != col[c]) {
+                seen[o] = col[c];
+                (col[o] < col[c] ? cnt.lo : cnt.hi)++;
+            }
             const int64_t i = (int64_t)s * nc + t;
             for (int d = 0; d < dim; d++) nrm[i * dim + d] = c1side ? -P.fn[(int64_t)f * dim + d] : P.fn[(int64_t)f * dim + d];
             nb[i] = o < 0 ? -1 : ((o << 2) | (col[o] < col[c] ? 1 : 0) | (col[o] > col[c] ? 2 : 0));
@@ -707,6 +717,7 @@ int build_colours(mst_ctx *x) {
     if (rc) return rc;
     x->lu_start = start;
     x->lu_colour = std::move(col);
+    x->lu_count = std::move(count);
     return MST_OK;
 }
 
@@ -1616,7 +1627,10 @@ int mst_algorithmic_bytes(const mst_ctx *ctx, int kernel, double *bytes) {
     // faces: c0, c1, info, FP64 normal; cells: the arithmetic state; order 2: face-cell offsets
     // (FP64: face centres, partner centres and cell centres) and limited gradients
     // order 2: the side records (each read once), the record indices, the raw c0 state of boundary faces
-    const double ninc = (double)ctx->n_inc, nbnd = (double)(ctx->nf - ctx->prep.P.n_interior);
+    const double ninc = (double)ctx->n_inc, n2 = (double)ctx->prep.P.n_interior, nbnd = nf - n2;
+    // a viscous stage's route (run_stage)
+    const bool visc_patch = ctx->viscous && ctx->visc_patch &&
+                            (ctx->resolved >= 0 ? ctx->resolved : ctx->strategy) != MST_STRATEGY_FACE;
     double flux_in = nf * (12 + 8 * D) + nc * r * NV;
     if (second) flux_in = nf * (12 + 8 * D + 8) + ninc * r * NV + nbnd * r * NV;
     // update: cell faces, stage state, volume, new state (+ FP32 shadow), Q^n on stages after the
@@ -1633,7 +1647,8 @@ int mst_algorithmic_bytes(const mst_ctx *ctx, int kernel, double *bytes) {
         case MST_K_GRAD:  // incidences: code, weight (not FP32 3D: folded into the normal), normal, offset,
                           // record out; cells: state, volume
             *bytes = 4.0 * ctx->slots * nc + ninc * (w_inc + 2 * r * D + r * NV) + nc * (r * NV + r);
-            if (ctx->viscous && ctx->visc_patch && !mixed) *bytes += nc * 8 * (D + 1) * D;  // viscous gradients out
+            // viscous gradients out; the kinds of boundary faces
+            if (visc_patch && second && !mixed) *bytes += nc * 8 * (D + 1) * D + nbnd * 8;
             break;
         case MST_K_UPDATE:
             *bytes = upd + nf * 8 * NV;
@@ -1645,7 +1660,7 @@ int mst_algorithmic_bytes(const mst_ctx *ctx, int kernel, double *bytes) {
             // (a face's kind comes with its packed list entry when there is one)
             *bytes = flux_in + upd - (mixed ? 0 : (second ? nbnd : nc) * 8 * NV) - ell +
                      4.0 * (double)ctx->n_psolve + 2.0 * ctx->slots * nc - (ctx->pfi ? 4.0 * nf : 0.0);
-            if (ctx->viscous) *bytes += nc * 8 * ((D + 1) * D + (second ? NV : 0)) + nf * 16;  // viscous terms' inputs
+            if (ctx->viscous) *bytes += nc * 8 * (D + 1) * D + n2 * 8;  // viscous gradients, eta of faces of two cells
             break;
         case MST_K_FUSED: {  // gradient inputs + per-face inputs + update, each once; no records
             // per incidence: code, weight, offset, and in 3D the normal (2D takes it from its face's)
@@ -1658,28 +1673,42 @@ int mst_algorithmic_bytes(const mst_ctx *ctx, int kernel, double *bytes) {
         case MST_K_DT:
             *bytes = nc * (8 * NV + 8 + 8 * D);
             break;
-        case MST_K_VISC: {  // the gradient kernel and the face kernel, averaged over the two launches
+        case MST_K_VISC: {
             const double nw = D + 1;
-            const double grad = 4.0 * ctx->slots * nc + ninc * (8 + 8 * D) + nc * (8 * NV + 8 + 8 * nw * D);
-            const double face = nf * (8 + 8 + 8 * D + 2 * 8 * NV) + nc * (8 * NV + 8 * nw * D);
-            *bytes = 0.5 * (grad + face);
+            const double grad = 4.0 * ctx->slots * nc + ninc * (8 + 8 * D) + nbnd * 8 + nc * (8 * NV + 8 + 8 * nw * D);
+            const double face = nf * (8 + 4 + 8 * D + 2 * 8 * NV) + n2 * 8 + nc * (8 * NV + 8 * nw * D);
+            // face route: the gradient kernel and the face kernel, averaged over the two launches
+            *bytes = visc_patch ? grad : 0.5 * (grad + face);
             break;
         }
         case MST_K_LUSGS: {  // one iteration's sweeps, each array once per sweep, over their launches
-            if (ctx->lu_start.size() < 2) return mst::fail(MST_E_ARG, "no LU-SGS iteration has run");
+            if (ctx->lu_count.empty()) return mst::fail(MST_E_ARG, "no LU-SGS iteration has run");
             // 2 K - 1 launches for K colours; 2 K - 2 where colour 0's sweeps of consecutive
             // iterations run fused (the iterations of a call before its last)
-            const double K = (double)(ctx->lu_start.size() - 1);
-            const double S = ctx->slots, launches = (ctx->lu_inline && K >= 2) ? 2.0 * K - 2 : 2.0 * K - 1;
-            // forward: positions, residual, states, neighbour updates, update out, D out; per slot the
-            // record (neighbour code, normal) and r out.  backward: positions, D, states, updates in
-            // and out, new state; per slot the record and r.
-            double fwd = nc * (4 + 8 * NV * 4 + 8) + S * nc * (4 + 8 * D + 8);
-            // forward sweeps that compute the residual read each slot's face code and face info
-            // instead of the residual array
-            if (ctx->lu_inline) fwd += S * nc * 8 - nc * 8 * NV;
-            const double bwd = nc * (4 + 8 + 8 * NV * 4) + S * nc * (4 + 8 * D + 8);
-            *bytes = (fwd + bwd) / launches;
+            const int K = (int)ctx->lu_count.size();
+            const bool bf = ctx->lu_inline && K >= 2;
+            const double S = ctx->slots, v = 8 * NV;
+            double total = 0;
+            for (int k = 0; k < K; k++) {
+                const LuCount &l = ctx->lu_count[k];
+                const double n = (double)l.n, inc = (double)l.inc, lo = (double)l.lo, hi = (double)l.hi;
+                const double hinc = (double)l.inc_hi;
+                const double rec = n * 4 + 4 * std::min(S * n, inc + n);  // positions, neighbour codes
+                const bool last = k == K - 1;
+                // forward: records, residual (or the face words to compute it from), normals, states of the cells and
+                // their neighbours, lower neighbours' updates; update out, and radii and D, or the last colour's state
+                if (k > 0 || !bf)
+                    total += rec + n * (ctx->lu_inline ? 4 : v) + inc * 8 * D + v * (n + 2 * lo + hi) + v * n +
+                             (last ? v * n : inc * 8 + n * 8);
+                // backward (not the last colour): records, D, states and updates of the cells and their higher
+                // neighbours with the normals and radii toward them; update and state out
+                if (!last && (k > 0 || !bf)) total += rec + n * 8 + hinc * (8 * D + 8) + 2 * v * (n + hi) + 2 * v * n;
+                // colour 0's backward and next forward sweep in one: the forward sweep's face words, the remaining
+                // normals, radii, D and update out besides; no second read of a neighbour, one update stored
+                if (k == 0 && bf)
+                    total += rec + n * 8 + n * 4 + inc * 8 * D + hinc * 8 + 2 * v * (n + hi) + 2 * v * n + inc * 8 + n * 8;
+            }
+            *bytes = total / (bf ? 2 * K - 2 : 2 * K - 1);
             break;
         }
         default:
