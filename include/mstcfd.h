@@ -377,14 +377,17 @@ int mst_mlp_set_data(mst_mlp *m, const float *X, const float *T, int64_t n);
 int mst_mlp_reset_optimizer(mst_mlp *m);
 /* steps of Adam (beta 0.9 / 0.999, eps 1e-8) on batches of `batch` samples drawn by a counter-based
  * hash of (step, row) (the whole set in order when batch >= n).  Networks of width <= 128 and n_out <= 32
- * take three launches a step.  Wider ones: use_graph: replay one captured step (dropped whenever the training set or a buffer it uses is replaced; launched directly instead
- * while a rocprofiler-sdk tool is loaded in the process).  loss: mean squared error of the last batch */
+ * take three launches a step.  Wider ones: use_graph: replay one captured step (dropped whenever the training
+ * set or a buffer it uses is replaced; launched directly instead while a rocprofiler-sdk tool is loaded in
+ * the process).  loss: mean squared error of the last batch */
 int mst_mlp_train(mst_mlp *m, int steps, int batch, double lr, int use_graph, double *loss);
 /* de-normalised outputs Y [n x n_out] of X [n x n_in] (host arrays) */
 int mst_mlp_forward(mst_mlp *m, const float *X, int64_t n, float *Y);
-/* per-dispatch timing of the network's kernels (start/stop HIP events carried by each launch; training
- * then launches directly instead of replaying its graph): count, summed milliseconds and summed
- * floating-point operations (GEMMs: 2 M N K) per kernel class */
+/* per-dispatch timing of the launch-per-layer kernels (start/stop HIP events carried by each launch): count, summed
+ * milliseconds and summed floating-point operations (GEMMs: 2 M N K) per kernel class.  While it is on, training
+ * launches directly instead of replaying its graph, and networks of width <= 128 and n_out <= 32 take these
+ * kernels too, in place of the three whole-network launches they run otherwise: the same bits, several times
+ * slower.  Their own speed is the time of mst_mlp_train with timing off. */
 #define MST_MLP_K_GEMM_FWD 0   /* forward GEMMs (bias + tanh epilogues) */
 #define MST_MLP_K_GEMM_WGRAD 1 /* weight-gradient GEMMs (batch split) */
 #define MST_MLP_K_GEMM_DGRAD 2 /* activation-gradient GEMMs (tanh' epilogue) */

@@ -744,7 +744,7 @@ class MLP:
         return loss.value
 
     def timing(self, on=True):
-        """Per-dispatch timing of the network's kernels (training launches directly while it is on)."""
+        """Per-dispatch timing of the launch-per-layer kernels (every width runs them, launched directly, while it is on)."""
         _check(lib().mst_mlp_timing_enable(self.h, 1 if on else 0), "mst_mlp_timing_enable")
 
     def timing_get(self, kclass):
