@@ -362,7 +362,8 @@ int mst_batch_autotune(mst_batch *b, const char *cache_path, int force, int step
  * counterpart).  A fully connected network n_in -> width (tanh) x hidden_layers -> n_out (linear),
  * FP32, trained and evaluated by the library's own kernels.  Parameters: per layer W [out x in]
  * row-major, then b [out].  Features are normalised (f - in_shift) * in_scale, outputs de-normalised
- * y * out_scale + out_shift; the loss is the mean squared error of the de-normalised outputs. */
+ * y * out_scale + out_shift; the loss is the mean squared error of the de-normalised outputs.
+ * A network, like a context, takes one host thread at a time (no internal locking). */
 typedef struct mst_mlp mst_mlp;
 int mst_mlp_create(int n_in, int width, int hidden_layers, int n_out, uint64_t seed, mst_mlp **out);
 int mst_mlp_destroy(mst_mlp *m);

@@ -232,8 +232,10 @@ __device__ __forceinline__ float keep(float v, unsigned mask) { return __uint_as
 //   k_wgrad   every layer's weight-gradient products (64 x 64 tiles, split over the rows as k_gemm's grid.z
 //             is) and, in further blocks of the same grid, the partial column sums of the bias gradients
 //   k_adam_net  sums the splits, steps Adam and repacks the weights
-// What bounds them: v_mfma_f32_32x32x2_f32 takes 64 cycles of a SIMD, and the VALU's time (tanh) adds to it: FP32
-// matrix and vector instructions were not seen to overlap, within a wave or between two.  So the operands
+// What bounds them: v_mfma_f32_32x32x2_f32 takes 64 cycles of a SIMD, and most of the VALU's time (tanh) adds to it.
+// One matrix and 16 vector FP32 instructions, 27 and 28 ns each alone: 60 ns together in the only wave of a SIMD, 62 in
+// two waves with one kind each, 42 per wave where two or four waves have both; k_net has one wave per SIMD in training
+// (256 blocks of 32 rows) and two in inference.  So the operands
 // come in the order in which lanes consume them: weights from packed copies in matrix-fragment order (one
 // coalesced 16-byte load per lane feeds four instructions; the next layer's loads are issued before this
 // layer's products), activations from LDS in the same order.  (A branch-free tanh of 28 instructions was no
@@ -285,7 +287,7 @@ __device__ __forceinline__ void net_weights(const float *pack, int off, int slic
 
 // acc[t] = A(rows of tile t0 + t, :) B(:, the wave's 32 columns), k ascending; k8 <= KMAX.  FIXED (k8 = KMAX, a
 // multiple of 4): the activations of the next four groups are read during the products of these four.
-// beside(j) runs after group j's products are issued: other work for the time the matrix core takes.
+// beside(j) runs after group j's products are issued: other work between them.
 template <int MT, int NT, int KMAX, bool FIXED, typename F>
 __device__ __forceinline__ void net_mm(const float *lds, int t0, int k8, const float4 (&w)[NET_J], floatx16 (&acc)[NT],
                                        F beside) {
@@ -377,9 +379,9 @@ __global__ __launch_bounds__(GT, 2) void k_net(const NetArgs a) {
             if (l == 0) {
                 net_mm<MT, MT, NET_IN / 8, false>(buf[cur], 0, kin, w, acc, nothing);
             } else {
-                // the tiles after each other, the tanh of one beside the products of the next (a wave's
-                // VALU and matrix work overlap; the two waves of a SIMD, which pass the barriers
-                // together, would do both in step)
+                // the tiles after each other, the tanh of one between the products of the next: one tile's
+                // accumulators at a time, 108 registers against 128.  300,000 rows of 4 x 128: 407 us against 421
+                // with all products first; warm starts by networks of 2 x 16 to 8 x 128: 1 to 4 % shorter.
 #pragma unroll
                 for (int t = 0; t < MT; t++) {
                     floatx16 one[1];
@@ -484,8 +486,10 @@ __global__ __launch_bounds__(GT, 2) void k_net(const NetArgs a) {
     }
 }
 
-// LDS asked for (and not used) by a k_wgrad block: two blocks per CU, so that equal blocks spread evenly over the
-// CUs (4 x 128, 8192 rows: 23.4 us against 25.6 with up to four on a CU)
+// LDS asked for (and not used) by a k_wgrad block: at most two blocks per CU, so that equal blocks spread evenly over the
+// CUs.  Microseconds per training step, up to four on a CU / two: 4 x 128 53.4 / 53.2 (4,096 rows), 66.0 / 63.6 (8,192),
+// 108.6 / 99.6 (16,384), 368 / 347 (65,536); 8 x 128 92.4 / 91.2, 124.9 / 113.5, 203 / 181, 725 / 673; 3 x 96 51.0 /
+// 50.8 (8,192), 226 / 218 (65,536); 16 to 64 columns, and below 4,096 rows, the same within 1 %.
 constexpr int WGRAD_LDS = 56000;
 
 struct WgradArgs {
@@ -1127,8 +1131,7 @@ double sum_host(const float *dptr, int64_t n) {
 
 namespace mst {
 
-// later work of stream `after` waits for the earlier work of `before` (an event of its own per call: threads may share
-// a network)
+// later work of stream `after` waits for the earlier work of `before` (by an event of its own, which nothing keeps)
 static int follow(hipStream_t after, hipStream_t before) {
     if (after == before) return MST_OK;
     hipEvent_t ev = nullptr;
