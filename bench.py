@@ -580,8 +580,34 @@ def ramp_section(M, args, held_out=8):
                                 held_out=held_out, wall_s=time.perf_counter() - t0, cases=rows))
 
 
+def short_line(out):
+    """The default run's line without what makes it long (21,700 characters: more than a reader of a few KB of output
+    keeps): floats to 6 significant digits but for the headline, of each kernel the launches, mean time and rate, of each
+    strategy its step and dominant kernel, the warm start's summary without its cases.  --details keeps the whole."""
+    def r6(x):
+        if isinstance(x, dict):
+            if "kernels" in x:
+                x = dict(x, kernels={n: {k: t[k] for k in ("launches", "avg_us", "gbs") if k in t}
+                                     for n, t in x["kernels"].items()})
+            return {k: r6(v) for k, v in x.items()}
+        if isinstance(x, (list, tuple)):
+            return [r6(v) for v in x]
+        return float(f"{x:.6g}") if isinstance(x, float) else x
+
+    line = r6(out)
+    line.update((k, out[k]) for k in ("value", "ms_per_step") if k in out)
+    configs = line.get("configs", {})
+    for part in (line, configs.get("pulse3d", {})):
+        for st, v in part.get("strategies", {}).items():
+            r = v["roofline"]
+            part["strategies"][st] = dict(value=v["value"], ms_per_step=v["ms_per_step"], kernel=r["kernel"], frac=r["frac"])
+    configs.get("ramp", {}).get("warm_start", {}).pop("cases", None)
+    return line
+
+
 def main():
     ap = argparse.ArgumentParser()
+    ap.add_argument("--details", metavar="FILE", help="write the default run's full results there as JSON")
     ap.add_argument("--gpus", type=int, default=1)
     ap.add_argument("--steps", type=int, default=100)
     ap.add_argument("--warmup", type=int, default=10)
@@ -642,7 +668,10 @@ def main():
         print(f"bench: ramp done at {time.perf_counter() - t0:.0f} s", file=sys.stderr, flush=True)
         out["configs"] = dict(pulse3d=c3, ramp=c5)
     out["wall_s"] = time.perf_counter() - t0
-    print(json.dumps(out))
+    if args.details:
+        with open(args.details, "w") as f:
+            json.dump(out, f)
+    print(json.dumps(short_line(out)))
 
 
 if __name__ == "__main__":
