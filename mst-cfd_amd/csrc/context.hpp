@@ -89,10 +89,11 @@ struct mst_ctx {
     int dt_to = 0;           // the array that dt-reducing launches write
     // Patch and fused kernels with 2 BLOCK lanes per patch (the halo's gradients beside the patch's, the faces in one
     // pass): where the time is one patch's and not the chip's.  Microseconds per SSP-RK2 step, BLOCK / 2 BLOCK
-    // lanes, by patches: fused 2D 23.6 / 20.4 (32), 31.0 / 28.7 (512), 40 / 46 (704); fused 3D 47.6 / 39.8 (188),
-    // 66 / 76 (324); first-order patch 2D 14.0 / 13.3 (176), 16.6 / 16.6 (313), 21.9 / 23.5 (704); patch 3D
-    // 36 / 32 (41), 57.0 / 54.4 (324), 80.3 / 80.9 (633).
-    bool wide_patch = false, wide_fused = false;
+    // lanes, by patches: fused 2D triangles 23.6 / 20.4 (32), 31.0 / 28.7 (512), 40 / 46 (704); quadrilaterals FP64 31.4 /
+    // 26.4 (224), 39.7 / 46.4 (308), 44.5 / 52.7 (512) and mixed 26.6 / 22.5 (224), 34.0 / 31.0 (512), so up to one
+    // patch per CU in FP64 (run_fused_t); fused 3D 47.6 / 39.8 (188), 66 / 76 (324); first-order patch 2D 14.0 / 13.3
+    // (176), 16.6 / 16.6 (313), 21.9 / 23.5 (704); patch 3D 36 / 32 (41), 57.0 / 54.4 (324), 80.3 / 80.9 (633).
+    bool wide_patch = false;
     // Patches of SUB_PATCH cells where those of BLOCK cells would leave most of the chip idle: a stage's time is then
     // one patch's, and a patch of 64 cells is one wave of each phase's work on its compute unit instead of four (two in
     // a row on each SIMD).  One small patch per CU in 3D, two in 2D: beyond that their larger halo costs more.

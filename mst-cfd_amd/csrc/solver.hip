@@ -1012,7 +1012,6 @@ int mst_ctx_create(const mst_mesh *m, const mst_config *cfg, mst_ctx **out) {
     x->nblk_c = (x->nc + BLOCK - 1) / BLOCK;
     x->nblk_f = (x->nf + BLOCK - 1) / BLOCK;
     x->wide_patch = x->nblk_c <= (x->dim == 3 ? 512 : 256);
-    x->wide_fused = x->nblk_c <= (x->dim == 2 ? 512 : 256);
 #define TRY(e)            \
     do {                  \
         int _r = (e);     \

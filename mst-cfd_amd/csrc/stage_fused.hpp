@@ -43,13 +43,15 @@ int run_fused_t(mst_ctx *x, int mode, int is, int in, const Stage &sg, int iout)
                                 sizeof(double) * x->nv * (2 * BLOCK / 64));
     const bool roe = x->cfg.scheme == MST_SCHEME_ROE;
     const int lim = x->cfg.limiter;
+    // (the sweeps stand at mst_ctx::wide_patch)
+    const bool wide = x->nblk_c <= (DIM == 2 && (x->slots == 3 || std::is_same<T, float>::value) ? 512 : 256);
 #define MST_FUSED_L(SC, LM, MF)                                                                                         \
     if constexpr (has_sub_patches<DIM, T>()) if (x->patch_cells == SUB_PATCH)                                           \
         return launch_patch(x, MST_K_FUSED, k_fused<DIM, SC, LM, T, MF, SUB_PATCH, 2 * SUB_PATCH>, 2 * SUB_PATCH, shm,  \
                             ga, fa, a, pa, ha);                                                                         \
-    return x->wide_fused ? launch_patch(x, MST_K_FUSED, k_fused<DIM, SC, LM, T, MF, BLOCK, 2 * BLOCK>, 2 * BLOCK, shm,  \
-                                        ga, fa, a, pa, ha)                                                              \
-                         : launch_patch(x, MST_K_FUSED, k_fused<DIM, SC, LM, T, MF>, BLOCK, shm, ga, fa, a, pa, ha);
+    return wide ? launch_patch(x, MST_K_FUSED, k_fused<DIM, SC, LM, T, MF, BLOCK, 2 * BLOCK>, 2 * BLOCK, shm, ga, fa, a, \
+                               pa, ha)                                                                                  \
+                : launch_patch(x, MST_K_FUSED, k_fused<DIM, SC, LM, T, MF>, BLOCK, shm, ga, fa, a, pa, ha);
 #define MST_FUSED_S(SC, MF)                                                                   \
     if (lim == MST_LIM_NONE) { MST_FUSED_L(SC, MST_LIM_NONE, MF) }                            \
     if (lim == MST_LIM_MINMOD) { MST_FUSED_L(SC, MST_LIM_MINMOD, MF) }                        \
