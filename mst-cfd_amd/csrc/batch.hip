@@ -543,6 +543,7 @@ struct mst_batch {
     double lu_cfl = 1e4, lu_omega = 1.0;
     int32_t *lu_cells = nullptr, *lu_nb = nullptr, *lu_face = nullptr, *lu_pcase = nullptr, *lu_fcase = nullptr;
     uint32_t *lu_info = nullptr;
+    bool roe_only = true;  // no case runs AUSM
     double *lu_n = nullptr, *lu_r = nullptr, *lu_D = nullptr, *lu_dQ = nullptr;
     int64_t *lu_cstart = nullptr;
     uint8_t *lu_active = nullptr;
@@ -1219,6 +1220,18 @@ LuArgs lu_args_b(const mst_batch *b) {
     return a;
 }
 
+// Whether an iteration's residual is computed in its forward sweeps (lu_inline_run_b).  Half the launches, but each is a
+// chain of the residual's solves and the sweep's, and AUSM's is the longer one, longest where a batch has both schemes:
+// below the lines the flux kernel and the separate sweeps are faster.  Microseconds per iteration, in the sweeps /
+// separate, Roe, AUSM, both: 16,000 triangles 16.2 / 18.7, 18.4 / 18.9, 20.9 / 19.6; 80,000 19.2 / 23.4, 21.5 / 23.6,
+// 23.9 / 24.1; 12,800 quadrilaterals 18.7 / 19.5, 21.6 / 20.0, 25.3 / 20.7; 65,536 21.3 / 23.8, 24.6 / 24.6, 24.1 / 24.4;
+// 2,592 tetrahedra 23.4 / 21.8, 28.3 / 22.1, 31.5 / 23.1; 36,000 24.5 / 25.6, 29.0 / 26.5, 32.9 / 26.7; 105,456 30.9 /
+// 37.7, 36.1 / 39.0, 39.3 / 40.2; 384,000 82 / 100, 94 / 103, 90 / 102.
+bool lu_inline(const mst_batch *b) {
+    const int64_t least = !b->roe_only ? 65536 : (b->dim == 3 ? 32768 : 0);
+    return b->order == 1 && b->lu_start.size() >= 3 && b->NC >= least;
+}
+
 // n >= 1 consecutive iterations (order 1, two colours or more) with the residual computed in the forward sweeps and
 // colour 0's backward sweep fused with its next forward one: 2 K - 2 launches per iteration for K colours,
 // where the flux kernel and the separate sweeps take 2 K, and no face-flux array over all faces.  24 ramps of 7,680
@@ -1558,6 +1571,7 @@ int mst_batch_create(int n_cases, const mst_mesh *const *meshes, const mst_confi
         p64[i] = make_params<double>(c);
         p32[i] = make_params<float>(c);
         scheme[i] = c.scheme;
+        b->roe_only = b->roe_only && c.scheme == MST_SCHEME_ROE;
         gam[i] = c.gamma;
         cflv[i] = c.cfl;
         ncells[i] = (double)P.nc;
@@ -1770,7 +1784,7 @@ int mst_batch_lusgs_step(mst_batch *b, int n_iter) {
     HIPCHK(hipStreamSynchronize(b->stream));
     HIPCHK(hipMemcpy(b->lu_active, b->active.data(), b->n, hipMemcpyHostToDevice));
     int it = 0;
-    if (b->order == 1 && b->lu_start.size() >= 3 && n_iter > 1) {  // all but the last, which also gives the norms
+    if (lu_inline(b) && n_iter > 1) {  // all but the last, which also gives the norms
         it = n_iter - 1;
         rc = b->dim == 2 ? (b->slots == 3 ? lu_inline_run_b<2, 3>(b, it) : lu_inline_run_b<2, 4>(b, it))
                          : lu_inline_run_b<3, 4>(b, it);
