@@ -1588,28 +1588,29 @@ __global__ __launch_bounds__(FIN) void k_finish_min(const double *__restrict__ s
     }
 }
 
-// The W maxima of k_maxrel's partials (all >= 0, no NaN: any order) to the host's board in one block of NT lanes, eight
-// loads per field of each lane in flight together: n <= 8 NT is one round of the memory's latency, so MONITOR_GRID bounds
-// k_maxrel's partials by 8 FIN.  28 partials: 4 us where k_finish takes 8 and a stream synchronisation and a copy followed;
+// The W maxima of k_maxrel's partials (all >= 0, no NaN: any order) to the host's board in one block of NT lanes, U loads
+// per field of each lane in flight together: n <= U NT is one round of the memory's latency, so MONITOR_GRID bounds
+// k_maxrel's partials by 8 FIN.  (U = 1 up to two rounds: 0.5 us less than eight
+// loads that are mostly masked out.)  28 partials: 4 us where k_finish takes 8 and a stream synchronisation and a copy followed;
 // the whole call on 2M / 8M / 24.5M triangles: 35 / 113 / 287 us (41 / 143 / 440 with 256 lanes of one load each).
 constexpr int64_t MONITOR_GRID = 8 * FIN;
-template <int W, int NT>
+template <int W, int NT, int U>
 __global__ __launch_bounds__(NT) void k_finish_max(const double *__restrict__ part, int64_t n, Board *__restrict__ b,
                                                    uint32_t seq) {
     __shared__ double s[W][NT / 64];
     double v[W];
 #pragma unroll
     for (int k = 0; k < W; k++) v[k] = 0;
-    for (int64_t i = threadIdx.x; i < n; i += 8 * NT) {
-        double x[W][8];
+    for (int64_t i = threadIdx.x; i < n; i += U * NT) {
+        double x[W][U];
 #pragma unroll
         for (int k = 0; k < W; k++)
 #pragma unroll
-            for (int u = 0; u < 8; u++) x[k][u] = i + u * NT < n ? part[k * n + i + u * NT] : 0;
+            for (int u = 0; u < U; u++) x[k][u] = i + u * NT < n ? part[k * n + i + u * NT] : 0;
 #pragma unroll
         for (int k = 0; k < W; k++)
 #pragma unroll
-            for (int u = 0; u < 8; u++)
+            for (int u = 0; u < U; u++)
                 if (v[k] < x[k][u]) v[k] = x[k][u];
     }
 #pragma unroll

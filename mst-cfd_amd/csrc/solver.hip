@@ -632,10 +632,13 @@ int run_monitor(mst_ctx *x, double *out) {
                     x->part);
     if (rc) return rc;
     const uint32_t seq = ++x->board_seq;
-    if (n <= 8 * BLOCK)
-        hipLaunchKernelGGL((k_finish_max<NV, BLOCK>), dim3(1), dim3(BLOCK), 0, x->stream, (const double *)x->part, n, x->board, seq);
+    const double *part = x->part;
+    if (n <= 2 * BLOCK)
+        hipLaunchKernelGGL((k_finish_max<NV, BLOCK, 1>), dim3(1), dim3(BLOCK), 0, x->stream, part, n, x->board, seq);
+    else if (n <= 8 * BLOCK)
+        hipLaunchKernelGGL((k_finish_max<NV, BLOCK, 8>), dim3(1), dim3(BLOCK), 0, x->stream, part, n, x->board, seq);
     else
-        hipLaunchKernelGGL((k_finish_max<NV, FIN>), dim3(1), dim3(FIN), 0, x->stream, (const double *)x->part, n, x->board, seq);
+        hipLaunchKernelGGL((k_finish_max<NV, FIN, 8>), dim3(1), dim3(FIN), 0, x->stream, part, n, x->board, seq);
     HIPCHK(hipGetLastError());
     HIPCHK(board_wait(x->board, seq, x->stream));
     for (int k = 0; k < NV; k++) out[k] = x->board->mon[k];
