@@ -28,12 +28,6 @@ using namespace mstk;
 // blocks of BLOCK cells up to which patches are of SUB_PATCH cells, 2D and 3D (mst_ctx::patch_cells)
 constexpr int64_t SUB_PATCH_MAX[2] = {128, 64};
 
-// what the LU-SGS sweeps of one colour touch: its cells, their incidences (toward cells of a higher colour), and the
-// distinct neighbours of lower and of higher colour
-struct LuCount {
-    int64_t n = 0, inc = 0, inc_hi = 0, lo = 0, hi = 0;
-};
-
 // ====================================================================================== context
 struct mst_ctx {
     mst_prep prep;
@@ -120,7 +114,6 @@ struct mst_ctx {
     uint32_t *lu_info = nullptr;
     std::vector<int64_t> lu_start;
     std::vector<int32_t> lu_colour;  // per cell (host copy)
-    std::vector<LuCount> lu_count;   // per colour
     double *lu_n = nullptr, *lu_r = nullptr, *lu_D = nullptr, *lu_dQ = nullptr;
     int steady = MST_STEADY_EXPLICIT;
     double lu_cfl = 1e4, lu_omega = 1.0;

@@ -683,24 +683,14 @@ int build_colours(mst_ctx *x) {
     const int64_t slots = x->slots;
     std::vector<int32_t> nb(slots * nc, -2), fcode(slots * nc, -1);
     std::vector<double> nrm(slots * nc * dim, 0.0);
-    std::vector<LuCount> count(ncol);
-    std::vector<int32_t> seen(nc, -1);  // the colour that last counted the cell as a neighbour
     for (int64_t t = 0; t < nc; t++) {
         const int64_t c = cells[t];
-        LuCount &cnt = count[col[c]];
-        cnt.n++;
         for (int s = 0; s < P.maxf; s++) {
             const int32_t e = P.ell[(int64_t)s * nc + c];
             if (e < 0) break;
             const int32_t f = e >> 1;
             const bool c1side = e & 1;
             const int32_t o = c1side ? P.fc0[f] : P.fc1[f];
-            cnt.inc++;
-            if (o >= 0 && col[o] > col[c]) cnt.inc_hi++;
-            if (o >= 0 && col[o] != col[c] && seen[o] != col[c]) {
-                seen[o] = col[c];
-                (col[o] < col[c] ? cnt.lo : cnt.hi)++;
-            }
             const int64_t i = (int64_t)s * nc + t;
             for (int d = 0; d < dim; d++) nrm[i * dim + d] = c1side ? -P.fn[(int64_t)f * dim + d] : P.fn[(int64_t)f * dim + d];
             nb[i] = o < 0 ? -1 : ((o << 2) | (col[o] < col[c] ? 1 : 0) | (col[o] > col[c] ? 2 : 0));
@@ -720,8 +710,41 @@ int build_colours(mst_ctx *x) {
     if (rc) return rc;
     x->lu_start = start;
     x->lu_colour = std::move(col);
-    x->lu_count = std::move(count);
     return MST_OK;
+}
+
+// what the sweeps of each colour touch: its cells, their incidences (inc_hi: toward cells of a higher colour), and the
+// distinct neighbours of lower and of higher colour
+struct LuCount {
+    int64_t n = 0, inc = 0, inc_hi = 0, lo = 0, hi = 0;
+};
+
+std::vector<LuCount> lu_counts(const mst_ctx *x) {
+    const auto &P = x->prep.P;
+    const auto &col = x->lu_colour;
+    const int64_t nc = x->nc;
+    std::vector<LuCount> count(x->lu_start.size() - 1);
+    std::vector<int32_t> seen(nc, -1);  // the colour that last counted the cell as a neighbour
+    for (size_t k = 0; k < count.size(); k++) count[k].n = x->lu_start[k + 1] - x->lu_start[k];
+    for (int s = 0; s < P.maxf; s++)
+        for (int64_t c = 0; c < nc; c++) {
+            const int32_t e = P.ell[(int64_t)s * nc + c];
+            if (e < 0) continue;
+            const int32_t o = (e & 1) ? P.fc0[e >> 1] : P.fc1[e >> 1];
+            count[col[c]].inc++;
+            if (o >= 0 && col[o] > col[c]) count[col[c]].inc_hi++;
+        }
+    for (size_t k = 0; k < count.size(); k++)  // (a colour at a time: `seen` holds one)
+        for (int s = 0; s < P.maxf; s++)
+            for (int64_t c = 0; c < nc; c++) {
+                const int32_t e = col[c] == (int32_t)k ? P.ell[(int64_t)s * nc + c] : -1;
+                if (e < 0) continue;
+                const int32_t o = (e & 1) ? P.fc0[e >> 1] : P.fc1[e >> 1];
+                if (o < 0 || col[o] == (int32_t)k || seen[o] == (int32_t)k) continue;
+                seen[o] = (int32_t)k;
+                (col[o] < (int32_t)k ? count[k].lo : count[k].hi)++;
+            }
+    return count;
 }
 
 template <typename K>
@@ -1684,15 +1707,21 @@ int mst_algorithmic_bytes(const mst_ctx *ctx, int kernel, double *bytes) {
             break;
         }
         case MST_K_LUSGS: {  // one iteration's sweeps, each array once per sweep, over their launches
-            if (ctx->lu_count.empty()) return mst::fail(MST_E_ARG, "no LU-SGS iteration has run");
+            if (ctx->lu_start.size() < 2) return mst::fail(MST_E_ARG, "no LU-SGS iteration has run");
+            std::vector<LuCount> count;
+            try {
+                count = lu_counts(ctx);
+            } catch (const std::bad_alloc &) {
+                return mst::fail(MST_E_ARG, "out of host memory");
+            }
             // 2 K - 1 launches for K colours; 2 K - 2 where colour 0's sweeps of consecutive
             // iterations run fused (the iterations of a call before its last)
-            const int K = (int)ctx->lu_count.size();
+            const int K = (int)count.size();
             const bool bf = ctx->lu_inline && K >= 2;
             const double S = ctx->slots, v = 8 * NV;
             double total = 0;
             for (int k = 0; k < K; k++) {
-                const LuCount &l = ctx->lu_count[k];
+                const LuCount &l = count[k];
                 const double n = (double)l.n, inc = (double)l.inc, lo = (double)l.lo, hi = (double)l.hi;
                 const double hinc = (double)l.inc_hi;
                 const double rec = n * 4 + 4 * std::min(S * n, inc + n);  // positions, neighbour codes
