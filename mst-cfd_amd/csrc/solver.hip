@@ -930,8 +930,8 @@ int time_strategies(mst_ctx *x, const int *cand, int n, int rounds) {
 // Blocks up to which AUTO looks no further than the patch kernels, where a mesh has patch tables.  On 20 meshes of 2 to
 // 131,072 triangles, quadrilaterals and tetrahedra, both orders, schemes and precisions, viscous or not, a stage of the
 // face or the cell strategy took 1.03 to 1.65 times the better of patch and fused (mixed 3D AUSM on 10,368 cells: the
-// same, 14.7 us); at 140,000 to 162,000 cells 1.06 to 1.37.  So a first step of order 1 costs no trial there, and one
-// of order 2 14 stages: about 150 to 250 us, where timing all four strategies well enough took 600 to 1,500.
+// same, 14.7 us); at 140,000 to 162,000 cells 1.06 to 1.37.  So a first step of order 1, or in 3D FP64, costs no trial
+// there, and another of order 2 14 stages: about 150 us, where timing all four well enough took 600 to 1,500.
 constexpr int64_t AUTO_PATCH_MAX = 512;
 
 // AUTO: the strategy for this mesh and configuration.  Where more than one can be the fastest, a few stages of each are
@@ -952,7 +952,8 @@ int resolve_strategy(mst_ctx *x) {
             cand[n++] = MST_STRATEGY_CELL;
         }
         if (x->patch_ok) cand[n++] = MST_STRATEGY_PATCH;
-        if (x->fused_ok && x->cfg.order >= 2) cand[n++] = MST_STRATEGY_FUSED;  // (order 1: the patch kernel)
+        // (order 1: the patch kernel; small FP64 meshes in 3D: 1.00 to 1.39 times the patch kernels' time, so no trial)
+        if (x->fused_ok && x->cfg.order >= 2 && (!few || x->dim == 2 || x->mixed)) cand[n++] = MST_STRATEGY_FUSED;
     }
     x->resolved = cand[0];
     if (n > 1) {
