@@ -110,9 +110,9 @@ __global__ __launch_bounds__(NT) void kb_flux(const BArgs<T> a) {
 #pragma unroll
                 for (int k = 0; k < NV; k++) g[k] = 0;
             } else if (roe) {
-                face_flux<DIM, MST_SCHEME_ROE, SECOND, T>(fa, f, kind, mask, g);
+                face_flux<DIM, MST_SCHEME_ROE, SECOND, T, false>(fa, f, kind, mask, g);
             } else {
-                face_flux<DIM, MST_SCHEME_AUSM, SECOND, T>(fa, f, kind, mask, g);
+                face_flux<DIM, MST_SCHEME_AUSM, SECOND, T, false>(fa, f, kind, mask, g);
             }
             stq<NV>(fa.G + f * NV, g);
         }

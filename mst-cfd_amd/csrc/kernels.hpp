@@ -74,34 +74,7 @@ struct FluxArgs {
 // interior state and Y = its reconstructed face state for a boundary face, whose ghost combines the
 // two as the reference does.  Everything is read by face index, so the lanes of the two cells of a
 // face (cell strategy) load and then compute bit-identical states.
-template <int DIM, bool SECOND, typename T>
-__device__ __forceinline__ void face_load(const FluxArgs<T> &a, int64_t f, int kind, double (&n64)[DIM],
-                                          T (&X)[DIM + 2], T (&Y)[DIM + 2]) {
-    constexpr int NV = DIM + 2;
-#pragma unroll
-    for (int d = 0; d < DIM; d++) n64[d] = a.fn[f * DIM + d];
-    if (kind == mst::KIND_INTERIOR || kind == mst::KIND_PERIODIC) {
-        if constexpr (SECOND) {
-            ldq<NV>(a.rec + (int64_t)a.frec0[f] * NV, X);
-            ldq<NV>(a.rec + (int64_t)a.frec1[f] * NV, Y);
-        } else {
-            ldq<NV>(a.Q + (int64_t)a.fc0[f] * NV, X);
-            ldq<NV>(a.Q + (int64_t)a.fc1[f] * NV, Y);
-        }
-        return;
-    }
-    ldq<NV>(a.Q + (int64_t)a.fc0[f] * NV, X);
-    if constexpr (SECOND) {
-        ldq<NV>(a.rec + (int64_t)a.frec0[f] * NV, Y);
-    } else {
-#pragma unroll
-        for (int k = 0; k < NV; k++) Y[k] = X[k];
-    }
-}
-
-// The same from the face's entries s0, s1 of the side arrays (frec0, frec1 at order 2, else fc0, fc1), fetched before.  (As
-// the base of the form above, which then loads s0 ahead of its branch, it cost k_flux 3 to 8 % in the mixed form:
-// 33.6 / 36.4 us on 663,552 tetrahedra, 15.7 / 16.3 on 500,000 quadrilaterals.)
+// s0, s1: the face's entries of the side arrays (frec0, frec1 at order 2, else fc0, fc1), fetched before.
 template <int DIM, bool SECOND, typename T>
 __device__ __forceinline__ void face_load(const FluxArgs<T> &a, int64_t f, int kind, int32_t s0, int32_t s1,
                                           double (&n64)[DIM], T (&X)[DIM + 2], T (&Y)[DIM + 2]) {
@@ -121,6 +94,52 @@ __device__ __forceinline__ void face_load(const FluxArgs<T> &a, int64_t f, int k
 #pragma unroll
         for (int k = 0; k < NV; k++) Y[k] = X[k];
     }
+}
+
+// The same with the indices loaded here: ahead of the branch on the kind (c0's is fetched without waiting for the kind)
+// or inside it.  Neither is always the better one; measured in microseconds, ahead / inside, on 820,000 triangles and
+// 500,000 quadrilaterals (2D), 663,552 tetrahedra (3D), and batches of 300,000 triangles, 240,000 quadrilaterals and
+// 384,000 tetrahedra (kb_, per step):
+//   order 1: k_flux 17.4 / 18.5 (FP64), 13.0 / 13.6 (FP32); kb_flux 517 / 511; kb_patch 49.0 / 50.3
+//   order 2: k_flux 23.6 / 22.0 (FP64), 33.5 / 31.4 (FP32, 3D); kb_flux 490 / 466; kb_patch 171 / 165
+//   cells, FP64 2D: k_cell 38.2 / 40.3, 43.0 / 43.6 (orders 1, 2); kb_cell 375 / 402, 531 / 554
+//   cells, FP32 2D: k_cell 28.1 / 27.3, 33.7 / 32.2; kb_cell 357 / 337, 486 / 459
+//   cells, 3D: order 1 k_cell 46.3 / 48.3 (FP32), kb_cell 669 / 654; order 2 FP64 k_cell 92.7 / 87.5, kb_cell 1169 / 1037
+template <int DIM, bool SECOND, typename T, bool AHEAD = !SECOND>
+__device__ __forceinline__ void face_load(const FluxArgs<T> &a, int64_t f, int kind, double (&n64)[DIM],
+                                          T (&X)[DIM + 2], T (&Y)[DIM + 2]) {
+    constexpr int NV = DIM + 2;
+    const bool two = kind == mst::KIND_INTERIOR || kind == mst::KIND_PERIODIC;
+    if constexpr (AHEAD) {
+        const int32_t s0 = SECOND ? a.frec0[f] : a.fc0[f], s1 = two ? (SECOND ? a.frec1[f] : a.fc1[f]) : -1;
+        face_load<DIM, SECOND, T>(a, f, kind, s0, s1, n64, X, Y);
+    } else {
+#pragma unroll
+        for (int d = 0; d < DIM; d++) n64[d] = a.fn[f * DIM + d];
+        if (two) {
+            if constexpr (SECOND) {
+                ldq<NV>(a.rec + (int64_t)a.frec0[f] * NV, X);
+                ldq<NV>(a.rec + (int64_t)a.frec1[f] * NV, Y);
+            } else {
+                ldq<NV>(a.Q + (int64_t)a.fc0[f] * NV, X);
+                ldq<NV>(a.Q + (int64_t)a.fc1[f] * NV, Y);
+            }
+            return;
+        }
+        ldq<NV>(a.Q + (int64_t)a.fc0[f] * NV, X);
+        if constexpr (SECOND) {
+            ldq<NV>(a.rec + (int64_t)a.frec0[f] * NV, Y);
+        } else {
+#pragma unroll
+            for (int k = 0; k < NV; k++) Y[k] = X[k];
+        }
+    }
+}
+
+// face_load's AHEAD in the cell kernels
+template <int DIM, bool SECOND, typename T>
+constexpr bool cell_ahead() {
+    return DIM == 2 ? std::is_same<T, double>::value : !SECOND;
 }
 
 // Riemann left (A: c0 side) and right (B: c1 side or ghost) states from face_load's inputs; registers only
@@ -191,12 +210,12 @@ __device__ __forceinline__ void face_solve(const Params<T> &P, bool roe, int kin
 }
 
 // G_f of one face: load, then solve
-template <int DIM, int SCHEME, bool SECOND, typename T>
+template <int DIM, int SCHEME, bool SECOND, typename T, bool AHEAD = !SECOND>
 __device__ __forceinline__ void face_flux(const FluxArgs<T> &a, int64_t f, int kind, int mask, double (&g)[DIM + 2]) {
     constexpr int NV = DIM + 2;
     double n64[DIM];
     T X[NV], Y[NV];
-    face_load<DIM, SECOND, T>(a, f, kind, n64, X, Y);
+    face_load<DIM, SECOND, T, AHEAD>(a, f, kind, n64, X, Y);
     face_solve<DIM, SCHEME, T>(a.P, SCHEME == MST_SCHEME_ROE, kind, mask, n64, X, Y, g);
 }
 
@@ -803,7 +822,8 @@ __device__ __forceinline__ void cell_fluxes(const FluxArgs<T> &fa, const int32_t
                 const int info = fa.finfo[f];
                 kind[s] = info & 15;
                 mask[s] = info >> 4;
-                if (kind[s] < mst::KIND_NONE) face_load<DIM, SECOND, T>(fa, f, kind[s], n64[s], X[s], Y[s]);
+                if (kind[s] < mst::KIND_NONE)
+                    face_load<DIM, SECOND, T, cell_ahead<DIM, SECOND, T>()>(fa, f, kind[s], n64[s], X[s], Y[s]);
             }
         }
 #pragma unroll
@@ -823,7 +843,7 @@ __device__ __forceinline__ void cell_fluxes(const FluxArgs<T> &fa, const int32_t
             if (kind >= mst::KIND_NONE) continue;  // zero-flux face
             double n64[DIM];
             T X[NV], Y[NV];
-            face_load<DIM, SECOND, T>(fa, f, kind, n64, X, Y);
+            face_load<DIM, SECOND, T, cell_ahead<DIM, SECOND, T>()>(fa, f, kind, n64, X, Y);
             double g[NV];
             face_solve<DIM, SCHEME, T>(fa.P, roe, kind, info >> 4, n64, X, Y, g);
             accumulate<NV, F32>(r, cmp, g, e & 1);
